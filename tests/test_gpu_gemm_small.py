@@ -1,0 +1,128 @@
+"""GPU parity of the GEMM kernels where their tiles do not divide the product:
+gemm_small.hip's 32- and 64-wide tiles (LDS DMA, and the register path for
+sizes and alignments DMA does not take) and the DMA kernel's edge tiles,
+against float64 products (oracle.closed_form.matmul).
+
+Tolerance: each of K f32 additions rounds by at most 2^-24 of its partial sum;
+the signs are random, so the result is off by about sqrt(K) 2^-24 of its norm,
+and the bar is four times that.  i8 results are whole numbers and equal.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import xtile_amd as xt
+from oracle import bf16_bits_to_f32, closed_form, f32_to_bf16_bits
+from tests.conftest import oracle_threads
+from tests.gpu_util import frob_rel, run_gpu, run_oracle, to_device
+from xtile_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def _narrow(rng, shape, dt):
+    x = rng.uniform(-1, 1, shape).astype(np.float32)
+    return x.astype(np.float16) if dt == "f16" else f32_to_bf16_bits(x)
+
+
+def _wide(x):
+    return (bf16_bits_to_f32(x) if x.dtype == np.uint16 else x).astype(np.float64)
+
+
+def _bar(k):
+    return 4 * np.sqrt(k) * 2.0**-24
+
+
+@pytest.mark.parametrize(
+    "dt,m,n,k,tm,tn,family",
+    [("f16", 40, 40, 72, 40, 40, "staged"),        # DMA: one tile with edges, K tail of one chunk
+     ("bf16", 96, 200, 520, 48, 40, "staged"),     # DMA: K tail, N's last tile 8 wide
+     ("f16", 8, 8, 8, 8, 8, "staged"),             # the smallest DMA product
+     ("bf16", 26, 65, 61, 13, 13, "staged"),       # registers: one column in the last tile, odd K
+     ("f16", 9, 9, 9, 9, 9, "staged"),             # registers: one more than a chunk
+     ("f16", 95, 60, 146, 19, 20, "staged"),       # registers, several tiles
+     ("bf16", 16, 7, 64, 16, 7, "staged"),         # N below a chunk: the staged kernel itself
+     ("f16", 1000, 1000, 1000, 40, 40, "staged"),  # 64 x 64 tiles, DMA
+     ("bf16", 999, 1001, 333, 37, 13, "staged"),   # 64 x 64 tiles, registers
+     ("f16", 64, 64, 64, 64, 64, "gemm"),          # fewer stages than waves
+     ("bf16", 64, 320, 640, 64, 64, "gemm"),       # 32 x 32
+     ("f16", 192, 1088, 4160, 64, 64, "gemm"),     # 32 x 64
+     ("f16", 1024, 1024, 1024, 128, 128, "gemm"),  # 64 x 64
+     ("f16", 2880, 512, 640, 64, 64, "gemm"),      # 128 x 128, M edge
+     ("bf16", 2112, 4160, 320, 64, 64, "gemm")],   # 256 x 256, M and N edges
+)
+def test_products_no_tile_divides(cuda, dt, m, n, k, tm, tn, family):
+    mod = (K.matmul_f16 if dt == "f16" else K.matmul_bf16)(m, n, k, tm, tn)
+    assert xt.plan(mod)["kernel"].startswith(family)
+    rng = np.random.default_rng(m + n + k)
+    a, b = _narrow(rng, (m, k), dt), _narrow(rng, (k, n), dt)
+    got = run_gpu(mod, [a, b, np.full((m, n), np.nan, np.float32)], [dt, dt, "f32"], cuda, case=f"{dt} {m}x{n}x{k}")[2]
+    assert frob_rel(got, closed_form.matmul(_wide(a), _wide(b))) <= _bar(k)
+
+
+@pytest.mark.parametrize(
+    "m,n,k,tm,tn",
+    [(48, 40, 72, 16, 8), (33, 51, 49, 33, 17), (64, 128, 128, 64, 64), (32, 65, 16, 16, 13),
+     (128, 1088, 4096, 64, 64), (2112, 2240, 256, 64, 64)],
+)
+def test_i8_epilogue_products_no_tile_divides(cuda, m, n, k, tm, tn):
+    """* scale + bias, astype(int8): the oracle's bytes."""
+    mod = K.matmul_i8(m, n, k, tm, tn)
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-128, 128, (m, k), dtype=np.int8)
+    b = rng.integers(-128, 128, (k, n), dtype=np.int8)
+    s = (rng.uniform(0.5, 2.0, (1, n)) / (np.sqrt(k) * 100)).astype(np.float32)
+    bias = rng.uniform(-20, 20, (1, n)).astype(np.float32)
+    bufs = [a, b, np.full((m, n), 99, np.int8), s, bias]
+    got = run_gpu(mod, bufs, ["i8", "i8", "i8", "f32", "f32"], cuda, case=f"i8 {m}x{n}x{k}")[2]
+    assert np.array_equal(got, run_oracle(mod, bufs, oracle_threads())[2])
+
+
+@xt.kernel
+def _part_kernel(a, b, out, tm, tn, tk):
+    i = xt.bid(0)
+    j = xt.bid(1)
+    x = xt.load(a, index=(i, 1), shape=(tm, tk))
+    w = xt.load(b, index=(1, j), shape=(tk, tn), shared=1)
+    xt.store(out, index=(i, j), tile=xt.matmul(x, w))
+
+
+@pytest.mark.parametrize("tm,tn,k", [(24, 40, 96), (20, 15, 33)])
+def test_product_of_part_of_its_arrays(cuda, tm, tn, k):
+    """A's second K columns, B's second K rows and half of B's and C's columns:
+    origins, pitches and a region narrower than its arrays.  The rest of C
+    stays as it was."""
+    m, n = 3 * tm, 5 * tn
+    mod = xt.convert(_part_kernel, args=(xt.Array((m, 2 * k), xt.float16), xt.Array((2 * k, 2 * n), xt.float16),
+                                        xt.Array((m, 2 * n), xt.float32), tm, tn, k), grid=(3, 5, 1))
+    assert xt.plan(mod)["kernel"].startswith("staged") and " gemm k=" in xt.plan(mod)["kernel"]
+    rng = np.random.default_rng(7)
+    a, b = _narrow(rng, (m, 2 * k), "f16"), _narrow(rng, (2 * k, 2 * n), "f16")
+    c = np.full((m, 2 * n), 5.0, np.float32)
+    got = run_gpu(mod, [a, b, c], ["f16", "f16", "f32"], cuda, case=f"part {tm}x{tn}x{k}")[2]
+    assert frob_rel(got[:, :n], closed_form.matmul(_wide(a[:, k:]), _wide(b[k:, :n]))) <= _bar(k)
+    assert np.all(got[:, n:] == 5.0)
+
+
+def test_buffers_off_the_vector_alignment(cuda):
+    """A, B and C one element past an aligned address: the register path, and
+    element stores."""
+    import torch
+
+    m = n = k = 80
+    mod = K.matmul_f16(m, n, k, 40, 40)
+    rng = np.random.default_rng(8)
+    a, b = _narrow(rng, (m, k), "f16"), _narrow(rng, (k, n), "f16")
+
+    def shifted(x, dt):
+        flat = torch.zeros(x.size + 1, dtype=dt, device=cuda)
+        flat[1:] = to_device(x, "f16" if dt == torch.float16 else "f32", cuda).reshape(-1)
+        return flat[1:].view(x.shape)
+
+    dev = [shifted(a, torch.float16), shifted(b, torch.float16), shifted(np.zeros((m, n), np.float32), torch.float32)]
+    print("[gpu] unaligned buffers", flush=True)
+    xt.launch(mod, *dev)
+    torch.cuda.synchronize()
+    assert frob_rel(dev[2].cpu().numpy(), closed_form.matmul(_wide(a), _wide(b))) <= _bar(k)

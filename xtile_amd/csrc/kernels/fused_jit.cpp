@@ -162,6 +162,8 @@ hipError_t launch_fused(const xt::Plan& p, void* const* bufs, hipStream_t s, std
     why = "fused plan has no compiled kernel";
     return hipErrorInvalidValue;
   }
+  hipError_t ge = hipSuccess;
+  if (p.gemm_ragged && launch_gemm_ragged(p, bufs, s, ge)) return ge;
   const xt::VmPlan& vm = p.vm;
   if (vm.access.size() > 8) {
     why = "fused kernels take at most 8 memref accesses";

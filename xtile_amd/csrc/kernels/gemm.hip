@@ -17,33 +17,17 @@
 // and bias columns).  Blocks are independent (README.md:85-89), so both are
 // pure scheduling choices.
 //
-// Programs whose Blocks map onto 256 x 256, 256 x 128, 128 x 256 or 128 x 128
-// workgroup tiles run on gemm_dma_kernel (operands landed in LDS by DMA;
-// described where it is defined), whatever the element type and result:
-// 256 x 256 when its tiles fill the CUs (or are few enough to split K), else
-// the first smaller tile whose tiles fill them, else the one with the most
-// tiles (launch_gemm).  Blocks that map onto 64 x 64 tiles only run on
-// gemm_kernel, a template for BM x BN tiles (instantiated at 64 x 64):
-//   * 4 waves of (BM/2) x (BN/2), v_mfma_f32_32x32x16_{f16,bf16} or
-//     v_mfma_i32_32x32x32_i8.  Every fragment is 16 bytes per lane, so one
-//     K slice is 128 bytes of every row whatever the element type (64 f16/bf16
-//     or 128 i8 values) and the staging below moves bytes.
-//   * A rows (K-contiguous) go global -> VGPR -> LDS as 16-byte vectors.  B is
-//     N-contiguous in memory but the matrix cores want K-contiguous lanes, so
-//     each thread loads an 8(k) x 8(n) block of 16-bit values or a
-//     16(k) x 8(n) block of bytes and transposes it in registers (16-bit
-//     halves, or 4x4 byte transposes with v_perm_b32) into eight N rows.
-//   * LDS tiles are unpadded [rows][128 B] arrays whose 16-byte chunks are
-//     XOR-swizzled (chunk c of row r at c ^ swz(r)): fragment reads and the
-//     transposed B stores both run at the bank-conflict-free rate.
-//   * Two register staging sets keep two K slices in flight; sched_group_barrier
-//     interleaves every MFMA with at most one fragment read, one global load,
-//     one LDS store and two VALU ops.
+// 256 x 256, 256 x 128, 128 x 256 and 128 x 128 workgroup tiles run on
+// gemm_dma_kernel (operands landed in LDS by DMA; described where it is
+// defined), whatever the element type and result: 256 x 256 when the Blocks map
+// onto it and its tiles fill the CUs (or are few enough to split K), else the
+// first smaller tile whose tiles fill them.  Where none does, the rest compete
+// by estimated time (tile_us): the fullest of those tiles, 128 x 128 and 256 x
+// 256 tiles over the whole M x N region with the last ones reaching past it,
+// and gemm_small.hip's 64 x 64, 32 x 64 and 32 x 32 tiles, which also take the
+// products of any size and alignment (launch_gemm_ragged).
 //   * For an f32 result a half-wave stores one whole 128-byte line per
-//     accumulator register.  For an i8 result the MFMAs compute
-//     D = B^T-fragment x A-fragment instead, so each lane holds runs of four
-//     consecutive output columns of one row and writes them as one 4-byte
-//     store.
+//     accumulator register.
 //   * Workgroups are dispatched round-robin over the 8 XCDs; the linear id is
 //     remapped so that each XCD receives a contiguous run of tiles, and tiles
 //     are ordered in groups of GROUP tile columns so that concurrently resident
@@ -51,7 +35,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "common.h"
+#include "gemm_common.h"
 #include "launch.h"
 
 namespace xtk {
@@ -64,8 +48,6 @@ constexpr int SLICE = 128;  // bytes of K per LDS row and K slice
 constexpr int kDmaStages = 4;
 constexpr int kTileGroup = 8;  // tile columns per group of the workgroup order
 
-enum { kF16 = 0, kBF16 = 1, kI8 = 2 };
-
 // Waves of gemm_dma_kernel: 4 (one per SIMD, 128 x 128 each) or 8 (two per
 // SIMD, 128 x 64 each: half an LDS read more per MFMA, but a second wave to
 // issue MFMAs while one waits).  Measured in one call (bench.py, 2000
@@ -73,364 +55,6 @@ enum { kF16 = 0, kBF16 = 1, kI8 = 2 };
 // 317.2, C6 (i8) 72.6 and 71.2.
 template <int ELEM>
 constexpr int dma_waves() { return ELEM == kF16 ? 4 : 8; }
-
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef int int4v __attribute__((ext_vector_type(4)));
-typedef int int16v __attribute__((ext_vector_type(16)));
-
-struct GemmArgs {
-  const unsigned char* a;
-  const unsigned char* b;
-  void* c;
-  const float* scale;
-  const float* bias;
-  TileOff ta, tb, tc, ts, tbias;  // element offsets
-  long long lda, ldb, ldc;        // row pitches in elements
-  int nk;                         // K slices
-  int vgx, vgy;                   // virtual grid (fused axes divided by their factor)
-  int mul[3];                     // block id = virtual id * mul (fused axes)
-  int sub_m, sub_n;               // workgroup tiles per (fused) Block along M and N
-  int nwg;
-  int group;
-  int has_scale, has_bias;
-  // K split (DMA kernel, f32 results without an epilogue): nwg = tiles *
-  // ksplit workgroups, K range r covering stages [r S / ksplit, (r + 1) S /
-  // ksplit) of the S = 2 nk stages of 64 K bytes (ranges differ by at most
-  // one stage; kstages = the shortest); ksplit = 1, tiles = nwg otherwise
-  int tiles, ksplit, kstages;
-};
-
-template <int ELEM>
-struct Acc {
-  typedef float16v type;
-};
-template <>
-struct Acc<kI8> {
-  typedef int16v type;
-};
-
-template <int ELEM>
-__device__ __forceinline__ typename Acc<ELEM>::type mfma(uint4v a, uint4v b, typename Acc<ELEM>::type c) {
-  if constexpr (ELEM == kI8)
-    return __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(int4v, a), __builtin_bit_cast(int4v, b), c,
-                                                 0, 0, 0);
-  else if constexpr (ELEM == kBF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                   c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c,
-                                                  0, 0, 0);
-}
-
-// Workgroup -> tile origins.  Contiguous runs per XCD, then GROUP-wide column
-// groups over the virtual grid.
-struct TilePtrs {
-  const unsigned char* A;
-  const unsigned char* B;
-  long long c_off;  // element offset of the C tile
-  const float* S;
-  const float* Bias;
-};
-
-// The workgroup's linear id with contiguous runs per XCD: the K range is
-// gemm_lin / tiles, the tile gemm_lin % tiles.
-__device__ __forceinline__ int gemm_lin(const GemmArgs& p) {
-  int L = blockIdx.x;
-  if ((p.nwg & 7) == 0) L = (L & 7) * (p.nwg >> 3) + (L >> 3);
-  return L;
-}
-
-template <int ELEM, int BM, int BN, bool KS = false>
-__device__ __forceinline__ TilePtrs gemm_tile_of(const GemmArgs& p) {
-  constexpr int ES = ELEM == kI8 ? 1 : 2;
-  int L = gemm_lin(p);
-  if constexpr (KS) L -= (L / p.tiles) * p.tiles;
-  const int subs = p.sub_m * p.sub_n;
-  const int s = L % subs;
-  int blk = L / subs;
-  const int sm = s / p.sub_n;
-  const int sn = s - sm * p.sub_n;
-  const int per_plane = p.vgx * p.vgy;
-  const int vz = blk / per_plane;
-  blk -= vz * per_plane;
-  const int per_group = p.group * p.vgy;
-  const int gid = blk / per_group;
-  const int first = gid * p.group;
-  const int gsize = min(p.group, p.vgx - first);
-  const int r = blk - gid * per_group;
-  const int x = (first + r % gsize) * p.mul[0];
-  const int y = (r / gsize) * p.mul[1];
-  const int z = vz * p.mul[2];
-  TilePtrs t;
-  t.A = p.a + (p.ta.at(x, y, z) + (long long)sm * BM * p.lda) * ES;
-  t.B = p.b + p.tb.at(x, y, z) * ES + (long long)sn * BN * ES;
-  t.c_off = p.tc.at(x, y, z) + (long long)sm * BM * p.ldc + (long long)sn * BN;
-  t.S = p.scale + p.ts.at(x, y, z) + sn * BN;
-  t.Bias = p.bias + p.tbias.at(x, y, z) + sn * BN;
-  return t;
-}
-
-__device__ __forceinline__ int swz(int row) { return (row ^ (row >> 3)) & 7; }
-
-// 4x4 byte transpose: rows a..d (byte i = column i) -> o[i] = column i
-// (byte j = row j).  v_perm_b32 takes bytes 0-3 from its second and 4-7 from
-// its first source.
-__device__ __forceinline__ void transpose4x4(unsigned a, unsigned b, unsigned c, unsigned d, unsigned (&o)[4]) {
-  const unsigned ab_lo = __builtin_amdgcn_perm(b, a, 0x05010400u);  // a0 b0 a1 b1
-  const unsigned ab_hi = __builtin_amdgcn_perm(b, a, 0x07030602u);  // a2 b2 a3 b3
-  const unsigned cd_lo = __builtin_amdgcn_perm(d, c, 0x05010400u);
-  const unsigned cd_hi = __builtin_amdgcn_perm(d, c, 0x07030602u);
-  o[0] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x05040100u);  // a0 b0 c0 d0
-  o[1] = __builtin_amdgcn_perm(cd_lo, ab_lo, 0x07060302u);
-  o[2] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x05040100u);
-  o[3] = __builtin_amdgcn_perm(cd_hi, ab_hi, 0x07060302u);
-}
-
-// Global -> VGPR staging of one K slice and the VGPR -> LDS stores.  B
-// sub-blocks: nb = sb % (BN/8) selects 8 output columns, kb = sb / (BN/8) the
-// 16-byte chunk of K (8 values of 16 bits or 16 bytes).
-template <int ELEM, int BM, int BN>
-struct Stager {
-  static constexpr int AV = BM * 8 / 256;      // 16-byte A vectors per thread
-  static constexpr int NB = BN / 8;            // B column blocks
-  static constexpr int BSUB = 8 * NB;          // B sub-blocks per slice
-  static constexpr int BROWS = ELEM == kI8 ? 16 : 8;
-  static constexpr int KPS = ELEM == kI8 ? SLICE : SLICE / 2;  // K values per slice
-  uint4v ra[AV];
-  uint4v rb[ELEM == kI8 ? 1 : 8];  // 16-bit: 8 rows of 8 values
-  uint2v rb8[ELEM == kI8 ? 16 : 1];  // bytes: 16 rows of 8 values
-
-  // Buffer loads: the descriptors cover the workgroup's A and B panels, each
-  // lane keeps one 32-bit offset, and the per-slice / per-row parts travel as
-  // the uniform scalar offset, so the staging needs no per-row pointers.
-  // lda, ldb in bytes.
-  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t A, __amdgpu_buffer_rsrc_t B, unsigned lda,
-                                       unsigned ldb, int kt, int tid) {
-    const unsigned va = (unsigned)(tid >> 3) * lda + (tid & 7) * 16;
-#pragma unroll
-    for (int i = 0; i < AV; ++i)
-      ra[i] = __builtin_amdgcn_raw_buffer_load_b128(A, va, kt * SLICE + i * 32 * lda, 0);
-    if (BSUB >= 256 || tid < BSUB) {
-      const int nb = (unsigned)tid % NB, kb = (unsigned)tid / NB;
-      if constexpr (ELEM == kI8) {
-        const unsigned vb = (unsigned)(kb * 16) * ldb + nb * 8;
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          rb8[i] = __builtin_bit_cast(uint2v, __builtin_amdgcn_raw_buffer_load_b64(B, vb, (kt * KPS + i) * ldb, 0));
-      } else {
-        const unsigned vb = (unsigned)(kb * 8) * ldb + nb * 16;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) rb[i] = __builtin_amdgcn_raw_buffer_load_b128(B, vb, (kt * KPS + i) * ldb, 0);
-      }
-    }
-  }
-
-  __device__ __forceinline__ void store(unsigned char (*As)[SLICE], unsigned char (*Bs)[SLICE], int tid) const {
-#pragma unroll
-    for (int i = 0; i < AV; ++i) {
-      const int v = tid + i * 256;
-      const int row = v >> 3, cv = v & 7;
-      *reinterpret_cast<uint4v*>(&As[row][(cv ^ swz(row)) * 16]) = ra[i];
-    }
-    if (BSUB >= 256 || tid < BSUB) {
-      const int nb = (unsigned)tid % NB, kb = (unsigned)tid / NB;
-      if constexpr (ELEM == kI8) {
-        // rows k = 0..15 of columns n = 0..7 -> column n holds 16 K bytes
-        uint4v col[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            unsigned o[4];
-            transpose4x4(rb8[4 * q][h], rb8[4 * q + 1][h], rb8[4 * q + 2][h], rb8[4 * q + 3][h], o);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) col[4 * h + i][q] = o[i];
-          }
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-          const int r = nb * 8 + n;
-          *reinterpret_cast<uint4v*>(&Bs[r][(kb ^ swz(r)) * 16]) = col[n];
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          // columns n = 2j (low halves) and 2j+1 (high halves) of the 8 loaded rows
-          uint4v even, odd;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const unsigned lo = rb[2 * q][j], hi = rb[2 * q + 1][j];
-            even[q] = (lo & 0xFFFFu) | (hi << 16);
-            odd[q] = (lo >> 16) | (hi & 0xFFFF0000u);
-          }
-          const int r0 = nb * 8 + 2 * j, r1 = r0 + 1;
-          *reinterpret_cast<uint4v*>(&Bs[r0][(kb ^ swz(r0)) * 16]) = even;
-          *reinterpret_cast<uint4v*>(&Bs[r1][(kb ^ swz(r1)) * 16]) = odd;
-        }
-      }
-    }
-  }
-};
-
-// x * s + b as two separately rounded f32 operations.
-__device__ __forceinline__ float scale_bias(float x, float s, float b, bool hs, bool hb) {
-#pragma clang fp contract(off)
-  float t = hs ? x * s : x;
-  return hb ? t + b : t;
-}
-
-__device__ __forceinline__ int ftoi_i8(float v) {
-  if (v != v) return 0;
-  const float r = __builtin_rintf(v);  // round half to even
-  return (int)fminf(fmaxf(r, -128.f), 127.f);
-}
-
-// The same conversion in three instructions: v_rndne_f32 (half to even),
-// v_cvt_i32_f32 (saturates out-of-range values and infinities, converts NaN
-// to 0; issued as assembly because a C++ cast of such values is undefined),
-// v_med3_i32 (clamp to [-128, 127]).
-__device__ __forceinline__ int ftoi_i8_fast(float v) {
-  int i;
-  asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(__builtin_rintf(v)));
-  return min(max(i, -128), 127);
-}
-
-// Low bytes of four ints packed into one word (byte e from q[e]).
-__device__ __forceinline__ unsigned pack_i8x4(const int (&q)[4]) {
-  const unsigned lo = __builtin_amdgcn_perm((unsigned)q[1], (unsigned)q[0], 0x0c0c0400u);  // q0 q1 0 0
-  const unsigned hi = __builtin_amdgcn_perm((unsigned)q[3], (unsigned)q[2], 0x04000c0cu);  // 0 0 q2 q3
-  return lo | hi;
-}
-
-template <int ELEM, int BM, int BN, bool OUT_I8>
-__global__ __launch_bounds__(256, BM * BN >= 65536 ? 1 : 2) void gemm_kernel(GemmArgs p) {
-  constexpr int WM = BM / 2, WN = BN / 2;  // 2 x 2 waves
-  constexpr int MI = WM / 32, NI = WN / 32;
-  constexpr int KS = SLICE / 32;  // MFMA K steps per slice (32 bytes each: 16 f16 or 32 i8)
-  typedef typename Acc<ELEM>::type acc_t;
-  __shared__ __attribute__((aligned(16))) unsigned char As[2][BM][SLICE];
-  __shared__ __attribute__((aligned(16))) unsigned char Bs[2][BN][SLICE];
-
-  const TilePtrs t = gemm_tile_of<ELEM, BM, BN>(p);
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  Stager<ELEM, BM, BN> st0, st1;
-  acc_t acc[MI][NI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-
-  const int nk = p.nk;  // >= 1
-  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(t.A), (short)0,
-                                                                       (int)0xFFFFFFFF, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned char*>(t.B), (short)0,
-                                                                       (int)0xFFFFFFFF, 0x00020000);
-  const unsigned lda = (unsigned)(p.lda * (ELEM == kI8 ? 1 : 2)), ldb = (unsigned)(p.ldb * (ELEM == kI8 ? 1 : 2));
-  st0.load(ra, rb, lda, ldb, 0, tid);
-  st1.load(ra, rb, lda, ldb, min(1, nk - 1), tid);
-  st0.store(As[0], Bs[0], tid);
-  __syncthreads();
-  const int lrow = lane & 31;
-  uint4v af[2][MI], bfr[2][NI];
-  // 16-byte chunk of this lane's K values in step ks: 2*ks + lane/32
-  auto read_frags = [&](int buf, int ks, int set) {
-    const int c = ks * 2 + (lane >> 5);
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-      const int r = wm * WM + i * 32 + lrow;
-      af[set][i] = *reinterpret_cast<const uint4v*>(&As[buf][r][(c ^ swz(r)) * 16]);
-    }
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int r = wn * WN + j * 32 + lrow;
-      bfr[set][j] = *reinterpret_cast<const uint4v*>(&Bs[buf][r][(c ^ swz(r)) * 16]);
-    }
-  };
-  // One K slice: compute from LDS[cur], request slice kt+2 into `next2`, move
-  // slice kt+1 from `next1` into LDS[cur^1].  Branch-free: slice indices are
-  // clamped to the last slice, whose repeated copies land in the idle buffer.
-  auto slice = [&](int kt, Stager<ELEM, BM, BN>& next2, const Stager<ELEM, BM, BN>& next1) {
-    const int cur = kt & 1;
-    read_frags(cur, 0, 0);
-    next2.load(ra, rb, lda, ldb, min(kt + 2, nk - 1), tid);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      if (ks + 1 < KS) read_frags(cur, ks + 1, (ks + 1) & 1);
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-          acc[i][j] = OUT_I8 ? mfma<ELEM>(bfr[ks & 1][j], af[ks & 1][i], acc[i][j])
-                             : mfma<ELEM>(af[ks & 1][i], bfr[ks & 1][j], acc[i][j]);
-    }
-    next1.store(As[cur ^ 1], Bs[cur ^ 1], tid);
-    __builtin_amdgcn_sched_group_barrier(0x100, MI + NI, 0);
-#pragma unroll
-    for (int g = 0; g < MI * NI * KS; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // global load
-      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
-      __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-    }
-    __syncthreads();
-  };
-  int kt = 0;
-  for (; kt + 1 < nk; kt += 2) {
-    slice(kt, st0, st1);      // st1 holds slice kt+1; st0 now fetches kt+2
-    slice(kt + 1, st1, st0);  // st0 holds slice kt+2; st1 now fetches kt+3
-  }
-  if (kt < nk) slice(kt, st0, st1);
-
-  const bool hs = p.has_scale, hb = p.has_bias;
-  if constexpr (OUT_I8) {
-    // D = B^T x A per 32x32 tile: lane l holds output row m = l%32 of tile i
-    // and register v output column 8*(v/4) + 4*(l/32) + v%4 of tile j, so four
-    // consecutive columns pack into one 4-byte store.
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n0 = wn * WN + j * 32 + 8 * g + 4 * (lane >> 5);
-        float4v sv = {1.f, 1.f, 1.f, 1.f}, bv = {0.f, 0.f, 0.f, 0.f};
-        if (hs) sv = *reinterpret_cast<const float4v*>(t.S + n0);
-        if (hb) bv = *reinterpret_cast<const float4v*>(t.Bias + n0);
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-          const long long off = t.c_off + (long long)(wm * WM + i * 32 + lrow) * p.ldc + n0;
-          unsigned packed = 0;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float y = scale_bias((float)acc[i][j][4 * g + e], sv[e], bv[e], hs, hb);
-            packed |= (unsigned)(ftoi_i8(y) & 0xff) << (8 * e);
-          }
-          *reinterpret_cast<unsigned*>(static_cast<signed char*>(p.c) + off) = packed;
-        }
-      }
-  } else {
-    // D = A x B per 32x32 tile: lane l holds output column l%32 of tile j and
-    // register v row 8*(v/4) + 4*(l/32) + v%4 of tile i; a half-wave writes one
-    // whole 128-byte line per register.
-    const int orow = (lane >> 5) * 4;
-#pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int n = wn * WN + j * 32 + lrow;
-      const float sv = hs ? t.S[n] : 1.f, bv = hb ? t.Bias[n] : 0.f;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const long long off = t.c_off + (long long)(wm * WM + i * 32 + (v >> 2) * 8 + orow + (v & 3)) * p.ldc + n;
-          static_cast<float*>(p.c)[off] = scale_bias((float)acc[i][j][v], sv, bv, hs, hb);
-        }
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // 256 x 256 GEMM whose operands reach LDS by DMA (buffer_load ... lds): no
@@ -471,9 +95,14 @@ __global__ __launch_bounds__(256, BM * BN >= 65536 ? 1 : 2) void gemm_kernel(Gem
 //     LDS round trip.  A stage's DMA has NS - 2 stages of compute to land.
 //     The barrier is a bare s_barrier: __syncthreads' release fence would
 //     also wait for the DMA that should stay in flight.
-template <int ELEM, int NS, bool OUT_I8, bool EPI, int NW, bool KS = false, int BMT = 256, int BNT = 256>
+//   * EDGE: the tiles cover one M x N region whose size no tile divides.  Rows
+//     past M and column chunks past N are clamped to ones that exist, and
+//     their results are not stored.  (Odd multiples of 64, which had run on 64
+//     x 64 tiles: bf16 4864 x 2112 x 1280 73 -> 37 us, 1984 x 1408 x 8064 96 ->
+//     69, f16 3776 x 6656 x 256 97 -> 37, i8 4224 x 2752 x 2176 90 -> 37.)
+template <int ELEM, int NS, bool OUT_I8, bool EPI, int NW, bool KS = false, int BMT = 256, int BNT = 256, bool EDGE = false>
 __global__ __launch_bounds__(64 * NW, BMT * BNT <= 128 * 128 ? 2 : 1) void gemm_dma_kernel(GemmArgs p) {
-  static_assert(!KS || (!EPI && !OUT_I8), "K split only without an epilogue");
+  static_assert(!KS || (!EPI && !OUT_I8 && !EDGE), "K split only without an epilogue");
   static_assert(NS >= 3 && NS <= 5, "stages");
   static_assert(NW == 4 || NW == 8, "waves");
   static_assert((BMT == 256 || BMT == 128) && (BNT == 256 || BNT == 128) && (NW == 4 || BMT * BNT == 65536),
@@ -501,16 +130,18 @@ __global__ __launch_bounds__(64 * NW, BMT * BNT <= 128 * 128 ? 2 : 1) void gemm_
   __shared__ __attribute__((aligned(1024))) unsigned char S4[NS > 4 ? STAGE : 16];
   unsigned char* const buf[5] = {S0, S1, S2, S3, S4};
 
-  const TilePtrs t = gemm_tile_of<ELEM, BM, BN, KS>(p);
+  int tx, ty;
+  const TilePtrs t = gemm_tile_of<ELEM, BM, BN, KS>(p, tx, ty);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / (NW / 2), wn = wave % (NW / 2);
   static_assert(WM * 2 == BM && WN * (NW / 2) == BN, "wave layout");
+  const int mleft = EDGE ? min(BM, p.M - ty * BM) : BM, nleft = EDGE ? min(BN, p.N - tx * BN) : BN;
   const i32x4 ra = raw_rsrc(t.A), rb = raw_rsrc(t.B);
   const unsigned lda = (unsigned)(p.lda * ES), ldb = (unsigned)(p.ldb * ES);
   // this workgroup's stages of 64 K bytes: [kbase, kbase + nk)
-  const int krange = KS ? gemm_lin(p) / p.tiles : 0;
+  const int krange = KS ? (int)p.d_tiles(gemm_lin(p)) : 0;
   const int kbase = KS ? (int)((long long)krange * (p.nk * 2) / p.ksplit) : 0;
   const int nk = KS ? (int)((long long)(krange + 1) * (p.nk * 2) / p.ksplit) - kbase : p.nk * 2;
 
@@ -524,12 +155,20 @@ __global__ __launch_bounds__(64 * NW, BMT * BNT <= 128 * 128 ? 2 : 1) void gemm_
   // (h, pc) = (L / CPR, L % CPR) holds chunk pc ^ bsw(RPI i + h), which
   // depends on i only through i & 1.
   constexpr int CPR = BR / 16;
-  const unsigned va = (unsigned)(lane >> 2) * lda + (unsigned)(((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  const unsigned ach = (unsigned)(((lane & 3) ^ ((lane >> 4) & 3)) << 4);
+  const unsigned va = (unsigned)(lane >> 2) * lda + ach;
+  unsigned va_edge[EDGE ? PA : 1];  // with the rows of this wave's instructions, clamped
+  if constexpr (EDGE)
+#pragma unroll
+    for (int q = 0; q < PA; ++q) va_edge[q] = (unsigned)min(16 * (wave * PA + q) + (lane >> 2), mleft - 1) * lda + ach;
   unsigned vb[2];
   {
     const int h = lane / CPR, pc = lane % CPR;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) vb[q] = (unsigned)h * ldb + (unsigned)((pc ^ bsw(RPI * q + h)) << 4);
+    for (int q = 0; q < 2; ++q) {
+      const int c = pc ^ bsw(RPI * q + h);
+      vb[q] = (unsigned)h * ldb + (unsigned)((EDGE && c * (16 / ES) >= nleft ? 0 : c) << 4);
+    }
   }
   // this wave's share of stage kt: A instructions PA w .. + PA - 1 (q < PA),
   // B instructions PB w .. + PB - 1 (q >= PA)
@@ -537,7 +176,8 @@ __global__ __launch_bounds__(64 * NW, BMT * BNT <= 128 * 128 ? 2 : 1) void gemm_
     const int kg = kt + kbase;
     if (q < PA) {
       const int i = wave * PA + q;
-      dma16(ra, lds_addr(S + i * 1024), va, (unsigned)(16 * i) * lda + (unsigned)kg * KB);
+      if constexpr (EDGE) dma16(ra, lds_addr(S + i * 1024), va_edge[q], (unsigned)kg * KB);
+      else dma16(ra, lds_addr(S + i * 1024), va, (unsigned)(16 * i) * lda + (unsigned)kg * KB);
     } else {
       const int i = wave * PB + (q - PA);
       dma16(rb, lds_addr(S + AB + i * 1024), vb[i & 1], (unsigned)(kg * KR + RPI * i) * ldb);
@@ -770,10 +410,12 @@ __global__ __launch_bounds__(64 * NW, BMT * BNT <= 128 * 128 ? 2 : 1) void gemm_
       for (int g = 0; g < 4; ++g) {
         const int n0 = wn * WN + j * 32 + 8 * g + 4 * hi;
         float4v sv = {1.f, 1.f, 1.f, 1.f}, bv = {0.f, 0.f, 0.f, 0.f};
+        if (EDGE && n0 >= nleft) continue;
         if (hs) sv = *reinterpret_cast<const float4v*>(t.S + n0);
         if (hb) bv = *reinterpret_cast<const float4v*>(t.Bias + n0);
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
+          if (EDGE && wm * WM + i * 32 + lrow >= mleft) continue;
           const long long off = t.c_off + (long long)(wm * WM + i * 32 + lrow) * p.ldc + n0;
           int q[4];
 #pragma unroll
@@ -793,12 +435,15 @@ __global__ __launch_bounds__(64 * NW, BMT * BNT <= 128 * 128 ? 2 : 1) void gemm_
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int n = wn * WN + j * 32 + lrow;
+      if (EDGE && n >= nleft) continue;
       const float sv = EPI && hs ? t.S[n] : 1.f, bv = EPI && hb ? t.Bias[n] : 0.f;
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const long long off = t.c_off + (long long)(wm * WM + i * 32 + (v >> 2) * 8 + orow + (v & 3)) * p.ldc + n;
+          const int m = wm * WM + i * 32 + (v >> 2) * 8 + orow + (v & 3);
+          if (EDGE && m >= mleft) continue;
+          const long long off = t.c_off + (long long)m * p.ldc + n;
           const float x = (float)acc[i][j][v];
           float* const o = static_cast<float*>(p.c) + off;
           // K split (never with an epilogue): the ranges' partial sums meet
@@ -874,72 +519,90 @@ __global__ __launch_bounds__(256) void gemm_zero_kernel(float* __restrict__ c, l
   __builtin_nontemporal_store(float4v{0.f, 0.f, 0.f, 0.f}, reinterpret_cast<float4v*>(c + r * ld) + q);
 }
 
-// The C tiles of all Blocks form one [M][N] region at c0 with pitch ld:
-// along one grid axis the Blocks step A and C by TM rows (B fixed), along
-// the other B and C by TN columns (A fixed).
-bool c_region(const xt::Plan& p, long long& M, long long& N) {
-  if (p.grid[2] != 1) return false;
-  const long long TM = p.a.rows, TN = p.b.cols;
-  for (int am = 0; am < 2; ++am) {
-    const int an = 1 - am;
-    const bool m_ok = p.grid[am] == 1 || (axis_step(p.a.addr, am) == TM * p.a.ld &&
-                                          axis_step(p.c.addr, am) == TM * p.c.ld && axis_step(p.b.addr, am) == 0);
-    const bool n_ok = p.grid[an] == 1 || (axis_step(p.b.addr, an) == TN && axis_step(p.c.addr, an) == TN &&
-                                          axis_step(p.a.addr, an) == 0);
-    if (m_ok && n_ok) {
-      M = TM * p.grid[am];
-      N = TN * p.grid[an];
-      return true;
-    }
+template <int ELEM, bool OUT_I8, int BMT, int BNT, bool EDGE>
+void launch_dma(const GemmArgs& a, hipStream_t s) {
+  constexpr int NW = BMT * BNT != 65536 ? 4 : EDGE ? 8 : dma_waves<ELEM>();  // EDGE with four waves spills
+  const dim3 grid(a.nwg), block(64 * NW);
+  if constexpr (OUT_I8) {
+    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, true, true, NW, false, BMT, BNT, EDGE>), grid, block, 0, s, a);
+  } else if (a.has_scale || a.has_bias) {
+    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, true, NW, false, BMT, BNT, EDGE>), grid, block, 0, s, a);
+  } else if (a.ksplit > 1) {
+    // the split is taken at square tiles without edges only
+    if constexpr (BMT == BNT && !EDGE)
+      hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, false, NW, true, BMT, BNT>), grid, block, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, false, NW, false, BMT, BNT, EDGE>), grid, block, 0, s, a);
   }
-  return false;
-}
-
-// The DMA kernel at a tile smaller than 256 x 256 (four waves).
-template <int ELEM, bool OUT_I8, int BMT, int BNT>
-void launch_small_t(const GemmArgs& a, hipStream_t s) {
-  const dim3 grid(a.nwg), block(256);
-  if constexpr (OUT_I8)
-    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, true, true, 4, false, BMT, BNT>), grid, block, 0, s, a);
-  else if (a.has_scale || a.has_bias)
-    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, true, 4, false, BMT, BNT>), grid, block, 0, s, a);
-  else if (BMT == 128 && BNT == 128 && a.ksplit > 1)
-    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, false, 4, true, 128, 128>), grid, block, 0, s, a);
-  else
-    hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, false, 4, false, BMT, BNT>), grid, block, 0, s, a);
 }
 
 template <int ELEM, bool OUT_I8>
 void launch_t(int bm, int bn, const GemmArgs& a, hipStream_t s) {
-  const dim3 grid(a.nwg), block(256);
-  if (bm == 256 && bn == 256) {
-    constexpr int NW = dma_waves<ELEM>();
-    const dim3 dblock(64 * NW);
-    if constexpr (OUT_I8)
-      hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, true, true, NW>), grid, dblock, 0, s, a);
-    else if (a.has_scale || a.has_bias)
-      hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, true, NW>), grid, dblock, 0, s, a);
-    else if (a.ksplit > 1)
-      hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, false, NW, true>), grid, dblock, 0, s, a);
-    else
-      hipLaunchKernelGGL((gemm_dma_kernel<ELEM, kDmaStages, false, false, NW>), grid, dblock, 0, s, a);
-  } else if (bm == 256) {
-    launch_small_t<ELEM, OUT_I8, 256, 128>(a, s);
-  } else if (bm == 128 && bn == 256) {
-    launch_small_t<ELEM, OUT_I8, 128, 256>(a, s);
-  } else if (bm == 128) {
-    launch_small_t<ELEM, OUT_I8, 128, 128>(a, s);
-  } else {
-    hipLaunchKernelGGL((gemm_kernel<ELEM, 64, 64, OUT_I8>), grid, block, 0, s, a);
-  }
+  if (bm == 256 && bn == 256)
+    a.edge ? launch_dma<ELEM, OUT_I8, 256, 256, true>(a, s) : launch_dma<ELEM, OUT_I8, 256, 256, false>(a, s);
+  else if (bm == 256)
+    launch_dma<ELEM, OUT_I8, 256, 128, false>(a, s);
+  else if (bn == 256)
+    launch_dma<ELEM, OUT_I8, 128, 256, false>(a, s);
+  else
+    a.edge ? launch_dma<ELEM, OUT_I8, 128, 128, true>(a, s) : launch_dma<ELEM, OUT_I8, 128, 128, false>(a, s);
 }
 
 }  // namespace
 
+// gemm_small.hip's tiles.  64 x 32 is not one: its 64-byte B rows are half cache
+// lines, and it measured behind 32 x 64 on every 16-bit product tried.
+static constexpr int kSmallTiles[3][2] = {{64, 64}, {32, 64}, {32, 32}};
+
+static int cu_count() {
+  int cus = 256, dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+    return 256;
+  return cus;
+}
+
+// Estimated microseconds of a launch of `tiles` bm x bn tiles (K in `ks`
+// ranges), fitted to graph-replay times of 30 products from 256 x 320 x 640 to
+// 3776 x 6656 x 256: a round of one tile a CU costs its start and end, its K
+// loop at the operand rate one CU reached, and its output at its share of HBM.
+// (64 x 64: 1024^3 f16 9.5 us measured, 9.2 estimated; 1024 x 1024 x 4096 21.0,
+// 20.1.  32 x 64: 256 x 2048 x 5632 18.9, 19.1.  32 x 32: 512^3 4.1, 4.7.
+// 128 x 128: 1536^2 x 4096 35.1, 37.)
+static double tile_us(int bm, int bn, long long tiles, long long ks, long long kbytes, long long es, int out_bytes, int cus) {
+  const bool bytes = es == 1;
+  double start, rate;  // us a round; KB of operands a us
+  if (bm >= 128) start = bm == 256 ? 3 : 2.5, rate = ks > 1 || bm == 256 ? 50 : 62;
+  else if (bm == 64) start = 3.2, rate = bytes ? 60 : 70;
+  else if (bn == 64) start = 2.1, rate = bytes ? 55 : 70;
+  else start = 1.5, rate = bytes ? 36 : 50;  // a row of B is a quarter or half of a cache line
+  const double round = start + double(bm + bn) * kbytes / ks / 1024 / rate + double(bm) * bn * out_bytes / 1024 / 30;
+  const double n = double(tiles) * ks / cus;
+  // 128 x 128 tiles run two to a CU, the others one
+  const double rounds = bm >= 128 && bm + bn < 512 && n > 2 ? n : std::ceil(n);
+  return 1.8 + rounds * round + (ks > 1 ? 2.8 + 2.0 * ks : 0);  // the zero fill, the atomic sums
+}
+
+// Tiles of bm x bn over the plan's whole M x N region, columns along x, rows
+// along y.
+static void region_tiles(const xt::Plan& p, long long M, long long N, int bm, int bn, GemmArgs& a) {
+  a.M = static_cast<int>(M);
+  a.N = static_cast<int>(N);
+  a.mul[0] = a.mul[1] = a.mul[2] = 1;
+  a.sub_m = a.sub_n = 1;
+  a.vgx = static_cast<int>((N + bn - 1) / bn);
+  a.vgy = static_cast<int>((M + bm - 1) / bm);
+  a.ta = TileOff{p.a.addr.c0, 0, bm * p.a.ld, 0};
+  a.tb = TileOff{p.b.addr.c0, bn, 0, 0};
+  a.tc = TileOff{p.c.addr.c0, bn, bm * p.c.ld, 0};
+  a.ts = TileOff{p.gemm_scale ? p.scale.addr.c0 : 0, bn, 0, 0};
+  a.tbias = TileOff{p.gemm_bias ? p.bias.addr.c0 : 0, bn, 0, 0};
+}
+
 hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std::string& why) {
   const bool i8 = p.a.elem == xt::Elem::I8;
   const long long es = i8 ? 1 : 2;
-  GemmArgs a;
+  GemmArgs a = {};
   a.a = static_cast<const unsigned char*>(bufs[p.a.arg]);
   a.b = static_cast<const unsigned char*>(bufs[p.b.arg]);
   a.c = bufs[p.c.arg];
@@ -990,24 +653,23 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
       return hipErrorInvalidValue;
     }
   }
-  int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-    cus = 256;
+  const int cus = cu_count();
   const bool out_i8 = p.c.elem == xt::Elem::I8;
-  long long M = 0, N = 0;
+  int64_t M = 0, N = 0;
   float* const cbase = static_cast<float*>(bufs[p.c.arg]) + p.c.addr.c0;
-  const bool can_split = ksplit_allowed() && !i8 && !out_i8 && !p.gemm_scale && !p.gemm_bias && c_region(p, M, N) && N % 4 == 0 &&
+  const bool region = xt::gemm_region(p, M, N) && M < (1LL << 31) && N < (1LL << 31);
+  const bool can_split = ksplit_allowed() && !i8 && !out_i8 && !p.gemm_scale && !p.gemm_bias && region && N % 4 == 0 &&
                          p.c.ld % 4 == 0 && reinterpret_cast<uintptr_t>(cbase) % 16 == 0 && M < (1LL << 31);
   // Workgroup tile, all on the DMA kernel: 256 x 256 when the Blocks map onto
   // it and its tiles fill the CUs, or are few enough for the K split below;
   // else the first of 256 x 128, 128 x 256, 128 x 128 whose tiles fill the
   // CUs, else the one with the most tiles (a 2048^3 f16 GEMM: 64 tiles of
-  // 256 x 256, 256 of 128 x 128); 64 x 64 (register-staged) when none maps.
+  // 256 x 256, 256 of 128 x 128).
   struct Cand {
     int bm = 0, bn = 0;
     Cover cm, cn;
     long long tiles = 0;
+    bool edge = false;  // tiles of the whole region, the last ones reaching past it
   };
   auto try_tile = [&](int bmv, int bnv, Cand& c) {
     c.bm = bmv;
@@ -1046,8 +708,39 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
       if (c.tiles > most.tiles) most = c;
     }
     if (!found) pick = most;
-    if (pick.bm == 0 && try_tile(64, 64, pick) == false) {
-      why = "matmul Blocks cannot be mapped onto 64x64 workgroup tiles";
+  }
+  // K ranges of the split below, 1 for none
+  auto ranges = [&](const Cand& c) {
+    const bool few = c.bm == 256 ? c.tiles * 8 <= cus : tiny && c.bm == 128 && c.tiles * 2 <= cus;
+    if (!can_split || c.edge || c.bm != c.bn || c.bm < 128 || !few) return 1LL;
+    return std::max(1LL, std::min<long long>(cus / c.tiles, a.nk * 2LL / 16));
+  };
+  // Where those tiles leave CUs idle, or none maps, the small tiles and the
+  // 128 x 128 and 256 x 256 tiles with edges compete by estimated time.
+  if (pick.bm == 0 || pick.tiles < cus) {
+    double best = pick.bm == 0 ? 1e30 : tile_us(pick.bm, pick.bn, pick.tiles, ranges(pick), kbytes, es, out_i8 ? 1 : 4, cus);
+    auto offer = [&](const Cand& c) {
+      const double us = tile_us(c.bm, c.bn, c.tiles, 1, kbytes, es, out_i8 ? 1 : 4, cus);
+      if (us < best && grid_fits(c.tiles, 512)) {
+        best = us;
+        pick = c;
+      }
+    };
+    for (const auto& sh : kSmallTiles) {
+      Cand c;
+      if (try_tile(sh[0], sh[1], c)) offer(c);
+    }
+    for (int t : {128, 256}) {
+      Cand c;
+      if (!region || try_tile(t, t, c) || t * a.lda * es >= (1LL << 32)) continue;
+      c = Cand{};
+      c.bm = c.bn = t;
+      c.edge = true;
+      c.tiles = (M + t - 1) / t * ((N + t - 1) / t);
+      offer(c);
+    }
+    if (pick.bm == 0) {
+      why = "matmul Blocks cannot be mapped onto workgroup tiles in one launch";
       return hipErrorInvalidValue;
     }
   }
@@ -1067,8 +760,10 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
   a.vgy = vg[1];
   a.sub_m = cm.sub;
   a.sub_n = cn.sub;
-  long long nwg = (long long)vg[0] * vg[1] * vg[2] * a.sub_m * a.sub_n;
-  if (!grid_fits(nwg, 256)) {
+  a.edge = pick.edge;
+  if (pick.edge) region_tiles(p, M, N, bm, bn, a);
+  long long nwg = pick.edge ? (long long)a.vgx * a.vgy : (long long)vg[0] * vg[1] * vg[2] * a.sub_m * a.sub_n;
+  if (!grid_fits(nwg, bm == 256 && bn == 256 ? 512 : 256)) {
     why = "matmul grid of " + std::to_string(nwg) + " workgroup tiles exceeds one launch";
     return hipErrorInvalidValue;
   }
@@ -1087,17 +782,19 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
   // Measured (f16, 30 launches): 1024 x 1024 x 4096 (16 tiles) 79.2 us whole,
   // 42.8 in 8 ranges; 2048^3 (64 tiles) 47.3 whole, 71.4 in 4; 1024 x 8192 x
   // 8192 (128 tiles) 155.9 whole, 164.4 in 2.
-  if (can_split && ((bm == 256 && bn == 256 && nwg * 8 <= cus) || (tiny && bm == 128 && bn == 128 && nwg * 2 <= cus))) {
-    const long long nk2 = a.nk * 2LL;
-    const long long ks = std::min<long long>(cus / nwg, nk2 / 16);
-    if (ks > 1) {
-      a.kstages = (int)(nk2 / ks);
-      a.ksplit = (int)ks;
-      a.nwg = (int)(nwg * ks);
-      const long long n4 = M * (N / 4);
-      hipLaunchKernelGGL(gemm_zero_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, cbase, p.c.ld,
-                         (int)M, (int)(N / 4));
-    }
+  if (const long long ks = ranges(pick); ks > 1) {
+    a.kstages = (int)(a.nk * 2LL / ks);
+    a.ksplit = (int)ks;
+    a.nwg = (int)(nwg * ks);
+    const long long n4 = M * (N / 4);
+    hipLaunchKernelGGL(gemm_zero_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, cbase, p.c.ld,
+                       (int)M, (int)(N / 4));
+  }
+  a.divide();
+  if (bm <= 64) {
+    a.K = static_cast<int>(p.gemm_k);
+    a.cvec = reinterpret_cast<uintptr_t>(static_cast<char*>(bufs[p.c.arg])) % 16 == 0;
+    return run_gemm_small(p.a.elem, out_i8, bm, bn, true, a, s);
   }
   switch (p.a.elem) {
     case xt::Elem::I8: out_i8 ? launch_t<kI8, true>(bm, bn, a, s) : launch_t<kI8, false>(bm, bn, a, s); break;
@@ -1107,6 +804,55 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
     default: out_i8 ? launch_t<kF16, true>(bm, bn, a, s) : launch_t<kF16, false>(bm, bn, a, s); break;
   }
   return hipGetLastError();
+}
+
+bool launch_gemm_ragged(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e) {
+  const bool i8 = p.a.elem == xt::Elem::I8, out_i8 = p.c.elem == xt::Elem::I8;
+  const long long es = i8 ? 1 : 2;
+  int64_t M, N;
+  if (!xt::gemm_region(p, M, N) || M >= (1LL << 31) || N >= (1LL << 31) || p.gemm_k >= (1LL << 17)) return false;
+  auto origin = [&](const xt::Access2D& v, long long b) { return static_cast<unsigned char*>(bufs[v.arg]) + v.addr.c0 * b; };
+  auto aligned = [](const void* q, long long n) { return reinterpret_cast<uintptr_t>(q) % n == 0; };
+  const unsigned char *A = origin(p.a, es), *B = origin(p.b, es), *C = origin(p.c, out_i8 ? 1 : 4);
+  if (!aligned(A, es) || !aligned(B, es) || (!out_i8 && !aligned(C, 4))) return false;
+  GemmArgs a = {};
+  a.a = static_cast<unsigned char*>(bufs[p.a.arg]);
+  a.b = static_cast<unsigned char*>(bufs[p.b.arg]);
+  a.c = bufs[p.c.arg];
+  if (p.gemm_scale) a.scale = static_cast<const float*>(bufs[p.scale.arg]);
+  if (p.gemm_bias) a.bias = static_cast<const float*>(bufs[p.bias.arg]);
+  if (!aligned(a.scale, 4) || !aligned(a.bias, 4)) return false;
+  a.has_scale = p.gemm_scale;
+  a.has_bias = p.gemm_bias;
+  a.lda = p.a.ld;
+  a.ldb = p.b.ld;
+  a.ldc = p.c.ld;
+  a.K = static_cast<int>(p.gemm_k);
+  a.edge = 1;
+  a.cvec = a.ldc % 4 == 0 && aligned(C, out_i8 ? 4 : 16);
+  const int cus = cu_count();
+  int bm = 0, bn = 0;
+  double best = 1e30;
+  for (const auto& sh : kSmallTiles) {
+    const double us = tile_us(sh[0], sh[1], (M + sh[0] - 1) / sh[0] * ((N + sh[1] - 1) / sh[1]), 1, p.gemm_k * es, es,
+                              out_i8 ? 1 : 4, cus);
+    if (us < best) best = us, bm = sh[0], bn = sh[1];
+  }
+  region_tiles(p, M, N, bm, bn, a);
+  const long long nwg = (long long)a.vgx * a.vgy;
+  if (!grid_fits(nwg, 256)) return false;
+  a.nwg = a.tiles = static_cast<int>(nwg);
+  a.ksplit = 1;
+  a.group = kTileGroup;
+  a.divide();
+  // LDS DMA: 16-byte rows and K chunks, and panels whose offsets stay below
+  // 2^31, where the K tail's out-of-range offsets begin
+  const bool dma = aligned(A, 16) && aligned(B, 16) && (a.lda * es) % 16 == 0 && (a.ldb * es) % 16 == 0 &&
+                   (a.K * es) % 16 == 0 && bm * a.lda * es < (1LL << 31) && a.K * a.ldb * es < (1LL << 31);
+  // the register path's loads of partial chunks reach back up to 16 bytes in a row
+  if (!dma && (a.K * es < 16 || N * es < 16)) return false;
+  e = run_gemm_small(p.a.elem, out_i8, bm, bn, dma, a, s);
+  return true;
 }
 
 }  // namespace xtk

@@ -62,6 +62,10 @@ hipError_t launch_ew_binary(const xt::Plan& p, void* const* bufs, hipStream_t s,
 hipError_t launch_row_softmax(const xt::Plan& p, void* const* bufs, hipStream_t s,
                               std::string& why);
 hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std::string& why);
+// A staged plan with gemm_ragged on the GEMM kernel for ragged sizes
+// (gemm_small.hip): false, with nothing launched, when the buffers or sizes are
+// outside what it takes; else `e` is the launch's status.
+bool launch_gemm_ragged(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e);
 hipError_t launch_conv2d(const xt::Plan& p, void* const* bufs, hipStream_t s, std::string& why);
 hipError_t launch_conv2d_general(const xt::Plan& p, void* const* bufs, hipStream_t s, std::string& why);
 // The implicit-GEMM conv kernel (conv_igemm.hip): false, with nothing

@@ -427,7 +427,8 @@ bool epilogue_row(const Analysis& an, const Op* bin, const Type& tile, Access2D&
   return access_of(an, *ld, acc, err);
 }
 
-bool match_gemm(const Analysis& an, Plan& p, std::string& err) {
+// ragged: any tile size and alignment.
+bool match_gemm_form(const Analysis& an, Plan& p, std::string& err, bool ragged) {
   int nmm, nst;
   const Op* mm = only(an, "xt.matmul", nmm);
   const Op* st = only(an, "xt.store", nst);
@@ -482,12 +483,12 @@ bool match_gemm(const Analysis& an, Plan& p, std::string& err) {
   }
   const bool i8 = ta.elem == Elem::I8;
   int64_t M = ta.shape[0], K = ta.shape[1], N = tb.shape[1];
-  if (M % 64 || N % 64 || K % (i8 ? 128 : 64)) {
+  if (!ragged && (M % 64 || N % 64 || K % (i8 ? 128 : 64))) {
     err = i8 ? "the HIP i8 matmul kernel needs tile M, N multiples of 64 and K a multiple of 128"
              : "the HIP matmul kernel needs tile M, N and K to be multiples of 64";
     return false;
   }
-  if (p.a.ld % (i8 ? 16 : 8) || p.b.ld % (i8 ? 16 : 8) || p.c.ld % 4) {
+  if (!ragged && (p.a.ld % (i8 ? 16 : 8) || p.b.ld % (i8 ? 16 : 8) || p.c.ld % 4)) {
     err = "the HIP matmul kernel needs 16-byte aligned rows";
     return false;
   }
@@ -507,6 +508,8 @@ bool match_gemm(const Analysis& an, Plan& p, std::string& err) {
   p.algo_bytes = bytes;
   return true;
 }
+
+bool match_gemm(const Analysis& an, Plan& p, std::string& err) { return match_gemm_form(an, p, err, false); }
 
 // -- Conv2d ----------------------------------------------------------------------
 
@@ -947,6 +950,7 @@ std::string Plan::describe() const {
     }
     case PlanKind::Fused:
       os << fused->layout << " insts=" << vm.inst.size();
+      if (gemm_ragged) os << " gemm k=" << gemm_k;
       break;
     case PlanKind::Conv2d:
       os << "conv2d_nhwc " << elem_name(conv.elem) << "->" << elem_name(conv.out_elem) << " tile=" << conv.TB
@@ -956,6 +960,27 @@ std::string Plan::describe() const {
   }
   os << " grid=(" << grid[0] << "," << grid[1] << "," << grid[2] << ")";
   return os.str();
+}
+
+bool gemm_region(const Plan& p, int64_t& M, int64_t& N) {
+  if (p.grid[2] != 1) return false;
+  const int64_t TM = p.a.rows, TN = p.b.cols;
+  auto step = [](const TileAddr& a, int axis) { return axis == 0 ? a.sx : a.sy; };
+  for (int am = 0; am < 2; ++am) {
+    const int n = 1 - am;
+    auto row_follows = [&](const Access2D& e) {
+      return (p.grid[am] == 1 || step(e.addr, am) == 0) && (p.grid[n] == 1 || step(e.addr, n) == TN);
+    };
+    const bool m_ok = p.grid[am] == 1 || (step(p.a.addr, am) == TM * p.a.ld && step(p.c.addr, am) == TM * p.c.ld &&
+                                          step(p.b.addr, am) == 0);
+    const bool n_ok = p.grid[n] == 1 || (step(p.b.addr, n) == TN && step(p.c.addr, n) == TN && step(p.a.addr, n) == 0);
+    if (m_ok && n_ok && (!p.gemm_scale || row_follows(p.scale)) && (!p.gemm_bias || row_follows(p.bias))) {
+      M = TM * p.grid[am];
+      N = TN * p.grid[n];
+      return true;
+    }
+  }
+  return false;
 }
 
 bool build_plan(const Module& m, const std::string& func, Plan& p, std::string& err) {
@@ -1034,6 +1059,22 @@ bool build_plan(const Module& m, const std::string& func, Plan& p, std::string& 
     std::string why, why_staged;
     if (!fuse_off && (fuse_vm(p.vm, p.grid, fp, why) ||
                       (!(stage_env && std::string(stage_env) == "0") && stage_vm(p.vm, p.grid, fp, why_staged)))) {
+      // a staged product whose sizes the GEMM form above refuses
+      Plan q = p;
+      std::string e2;
+      int64_t M, N;
+      if (fp.staged && match_gemm_form(an, q, e2, true) && gemm_region(q, M, N) && q.gemm_k < (int64_t(1) << 17)) {
+        p.a = q.a;
+        p.b = q.b;
+        p.c = q.c;
+        p.scale = q.scale;
+        p.bias = q.bias;
+        p.gemm_k = q.gemm_k;
+        p.gemm_scale = q.gemm_scale;
+        p.gemm_bias = q.gemm_bias;
+        p.gemm_ftoi = q.gemm_ftoi;
+        p.gemm_ragged = true;
+      }
       p.kind = PlanKind::Fused;
       p.fused = std::make_shared<FusedPlan>(std::move(fp));
       p.vm_fallback = vm_fits_interpreter(p.vm, p.vm_fallback_why);

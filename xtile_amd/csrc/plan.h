@@ -128,6 +128,10 @@ struct Plan {
   // row tiles, then an optional ftoi (the store's element type is then i8).
   bool gemm_scale = false, gemm_bias = false, gemm_ftoi = false;
   Access2D scale, bias;
+  // A staged program that is one product over a whole M x N region of C
+  // (gemm_region): a, b, c and the epilogue above describe it, and the GEMM
+  // kernel for ragged sizes runs it where the buffers allow.
+  bool gemm_ragged = false;
   ConvPlan conv;
   VmPlan vm;
   std::shared_ptr<FusedPlan> fused;  // Fused: the generated kernel (vm keeps the accesses)
@@ -155,6 +159,12 @@ bool fuse_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& out, std::strin
 // (LDS beyond 160 KB, more than 8 accesses, an exact matmul of values that
 // are not i8 tiles, a load of a memref the program stored to).
 bool stage_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& out, std::string& why, int max_vw = 4);
+
+// Whether the C tiles of a Gemm plan's Blocks form one [M][N] region at c0 with
+// pitch ld: along one grid axis the Blocks step A and C by a tile's rows (B and
+// the epilogue rows fixed), along the other B, C and the epilogue rows by a
+// tile's columns (A fixed).
+bool gemm_region(const Plan& p, int64_t& M, int64_t& N);
 
 // Builds the plan of function `func` (empty name: the only function).
 // Returns false and sets `error` when the program is not one the HIP
