@@ -95,6 +95,24 @@ int xt_plan(xt_module* m, const char* func, char** out_desc, double* algo_bytes,
 int xt_gpu_run(xt_module* m, const char* func, void* const* bufs, const size_t* buf_bytes,
                int nbufs, void* stream, char** err);
 
+/* Element types of xt_buffer. */
+typedef enum xt_dtype { XT_F32 = 0, XT_F16 = 1, XT_BF16 = 2, XT_I8 = 3, XT_I32 = 4 } xt_dtype;
+
+/* A dense row-major device buffer as its owner describes it. */
+typedef struct xt_buffer {
+  void* ptr;
+  const long long* shape;
+  int rank;
+  int dtype; /* xt_dtype */
+} xt_buffer;
+
+/* xt_gpu_run over described buffers: XT_ERR_ARGUMENT, with nothing launched,
+ * unless every buffer has its memref argument's element type and shape.  What
+ * the signature's JSON would tell the caller is checked here, so a launch
+ * needs no other call (no reference counterpart). */
+int xt_gpu_run_buffers(xt_module* m, const char* func, const xt_buffer* bufs, int nbufs, void* stream,
+                       char** err);
+
 #ifdef __cplusplus
 }
 #endif

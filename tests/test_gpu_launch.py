@@ -1,0 +1,88 @@
+"""xt.launch: the native call takes the plain case; everything else reaches the
+checked path, which launches it or raises the exception that names the fault."""
+
+from __future__ import annotations
+
+import pytest
+
+import xtile_amd as xt
+from xtile_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def _buffers(cuda):
+    import torch
+
+    a, b = torch.rand(64, 128, device=cuda), torch.rand(64, 128, device=cuda)
+    return a, b, torch.zeros(64, 128, device=cuda)
+
+
+@pytest.mark.parametrize("how", ["plain", "func", "int", "object", "current", "subclass"])
+def test_launches(cuda, monkeypatch, how):
+    import torch
+
+    m, (a, b, c) = K.add(64, 128), _buffers(cuda)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    checked = []
+    run = xt._launch_checked
+    monkeypatch.setattr(xt, "_launch_checked", lambda *x: (checked.append(how), run(*x)))
+    print(f"[gpu] launch {how}", flush=True)
+    if how == "func":
+        xt.launch(m, a, b, c, func="add_kernel")
+    elif how == "int":
+        xt.launch(m, a, b, c, stream=side.cuda_stream)
+    elif how == "object":
+        xt.launch(m, a, b, c, stream=side)
+    elif how == "current":
+        with torch.cuda.stream(side):
+            xt.launch(m, a, b, c)
+    elif how == "subclass":
+        class Wrapped(torch.Tensor):
+            pass
+
+        xt.launch(m, a.as_subclass(Wrapped), b, c)
+    else:
+        xt.launch(m, a, b, c)
+    torch.cuda.synchronize()
+    assert torch.equal(c, a + b)
+    assert checked == (["subclass"] if how == "subclass" else [])
+
+
+def test_refusals(cuda):
+    import torch
+
+    m, (a, b, c) = K.add(64, 128), _buffers(cuda)
+    with pytest.raises(ValueError, match="takes 3 buffers, got 2"):
+        xt.launch(m, a, b)
+    with pytest.raises(TypeError, match="buffer 1 must be a torch.Tensor"):
+        xt.launch(m, a, b.cpu().numpy(), c)
+    with pytest.raises(ValueError, match="buffer 2 is not on a GPU"):
+        xt.launch(m, a, b, c.cpu())
+    with pytest.raises(TypeError, match="buffer 0 has dtype torch.float16; expected f32"):
+        xt.launch(m, a.half(), b, c)
+    with pytest.raises(ValueError, match=r"buffer 1 has shape \(128, 64\); expected \(64, 128\)"):
+        xt.launch(m, a, b.reshape(128, 64), c)
+    with pytest.raises(ValueError, match="buffer 0 must be contiguous"):
+        xt.launch(m, torch.rand(128, 64, device=cuda).t(), b, c)
+    with pytest.raises(NotImplementedError):
+        xt.launch(K.add_rows(64, 128, 40), a, b, c)  # the last tile overruns
+    with pytest.raises(TypeError, match="expected an xtile module object"):
+        xt.launch(object(), a, b, c)
+    with pytest.raises(RuntimeError):  # a batched tensor has no data of its own
+        torch.func.vmap(lambda x: (xt.launch(m, x, b, c), x)[1])(torch.rand(2, 64, 128, device=cuda))
+    torch.cuda.synchronize()
+    assert not c.any()
+
+
+def test_a_pass_drops_the_plan(cuda):
+    """The plan a launch used is not kept across a pass over its module."""
+    import torch
+
+    m, (a, b, c) = K.add(64, 128), _buffers(cuda)
+    xt.launch(m, a, b, c)
+    xt.xt_serialize(m)
+    with pytest.raises((NotImplementedError, ValueError)):
+        xt.launch(m, a, b, c)
+    torch.cuda.synchronize()

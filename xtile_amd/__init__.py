@@ -187,10 +187,26 @@ def _torch_dtype(name: str):
     return _TORCH_DTYPES[name]
 
 
+_launch_native = None  # csrc/launch_torch.cpp's launch, loaded by the first one
+
+
 def launch(module: Any, *buffers, func: str | None = None, stream: Any = None) -> None:
     """Run `func` on the GPU.  `buffers` are torch tensors on one GPU, one per
     memref argument in argument order, contiguous, with the memref's dtype and
     shape.  Asynchronous on `stream` (default: torch's current stream)."""
+    global _launch_native
+    if _launch_native is None:
+        from ._compiled import load_launch
+
+        _launch_native = load_launch(_native)
+    handle = stream if stream is None else getattr(stream, "cuda_stream", stream)
+    if not _launch_native(getattr(module, "_CAPIPtr", module), buffers, func, handle):
+        _launch_checked(module, buffers, func, stream)
+
+
+def _launch_checked(module: Any, buffers: tuple, func: str | None, stream: Any) -> None:
+    """A launch the native call did not take: each condition by itself, with
+    the exception that names it, then the launch."""
     import torch
 
     sig = _native.signature(module, func)

@@ -41,3 +41,24 @@ def load():
         del sys.modules[MODULE_NAME]
         raise
     return module
+
+
+def load_launch(native):
+    """``launch`` of the compiled ``_launch`` module (``csrc/launch_torch.cpp``),
+    bound to the library that ``native``, the binding in use, parses modules
+    with.  ImportError when it is not built."""
+    import ctypes
+
+    import torch  # noqa: F401  (its libraries are the module's)
+
+    path = MODULE_PATH.with_name(MODULE_PATH.name.replace("_xtile", "_launch", 1))
+    if not path.exists():
+        raise ImportError(f"{path} is not built; run `python xtile_amd/build.py` (or __graft_entry__.build())")
+    spec = importlib.util.spec_from_file_location("xtile_amd.lib._launch", path)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    lib = getattr(native, "lib", None) or ctypes.CDLL(str(MODULE_PATH.with_name("libxtile_amd.so")))
+    module.bind(
+        ctypes.cast(lib.xt_gpu_run_buffers, ctypes.c_void_p).value, ctypes.cast(lib.xt_free, ctypes.c_void_p).value
+    )
+    return module.launch

@@ -80,6 +80,30 @@ SIGNATURES = {
 }
 
 
+class Buffer(ctypes.Structure):
+    """xt_buffer"""
+
+    _fields_ = [
+        ("ptr", ctypes.c_void_p),
+        ("shape", ctypes.POINTER(ctypes.c_longlong)),
+        ("rank", ctypes.c_int),
+        ("dtype", ctypes.c_int),
+    ]
+
+
+SIGNATURES["xt_gpu_run_buffers"] = (
+    ctypes.c_int,
+    [
+        ctypes.c_void_p,
+        ctypes.c_char_p,
+        ctypes.POINTER(Buffer),
+        ctypes.c_int,
+        ctypes.c_void_p,
+        ctypes.POINTER(ctypes.c_void_p),
+    ],
+)
+
+
 def _load() -> ctypes.CDLL:
     path = os.environ.get("XTILE_AMD_LIB", str(_LIB_PATH))
     if not os.path.exists(path):

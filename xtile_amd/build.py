@@ -7,6 +7,8 @@ Produces, under ``xtile_amd/lib/``:
   * ``_xtile<ext>.so``   - the compiled Python module ``_xtile``
     (``csrc/XTModule.cpp``, pybind11) over the C ABI, with the reference
     module's function names;
+  * ``_launch<ext>.so``  - ``xt.launch`` over torch tensors as one native call
+    (``csrc/launch_torch.cpp``, CPython and torch's C++ API);
   * ``libxt_ceiling.so`` - the measurement kernels of ``include/xt_ceiling.h``
     (a copy, an empty kernel and an MFMA loop) that bench.py times for its
     ceilings; the tile programs never use it.
@@ -92,6 +94,7 @@ def build(verbose: bool = False) -> Path:
     xt_opt_obj = OBJ / "xt_opt.o"
     jobs.append([CXX, *HOST_FLAGS, "-c", str(CSRC / "xt_opt.cpp"), "-o", str(xt_opt_obj)])
 
+    launch = ThreadPoolExecutor(max_workers=1).submit(build_launch)  # needs nothing of the rest
     workers = min(8, os.cpu_count() or 1)
     with ThreadPoolExecutor(max_workers=workers) as pool:
         for cmd in jobs:
@@ -123,6 +126,7 @@ def build(verbose: bool = False) -> Path:
     os.replace(ceil_tmp, LIB / "libxt_ceiling.so")
     _run([CXX, *map(str, host_objs), str(xt_opt_obj), "-o", str(LIB / "xt-opt")])
     build_module()
+    launch.result()
     return lib
 
 
@@ -151,6 +155,46 @@ def build_module() -> Path:
             f"-L{LIB}",
             "-lxtile_amd",
             "-Wl,-rpath,$ORIGIN",
+            "-o",
+            str(tmp),
+        ]
+    )
+    os.replace(tmp, out)
+    return out
+
+
+def launch_path() -> Path:
+    """Where build_launch() puts the ``_launch`` module."""
+    return LIB / ("_launch" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+
+
+def build_launch() -> Path:
+    """Compile csrc/launch_torch.cpp against the installed torch.  It is handed
+    the library's entry points at run time, so it links torch only."""
+    import torch
+    from torch.utils import cpp_extension
+
+    out = launch_path()
+    tmp = out.with_name(out.name + ".tmp")
+    _run(
+        [
+            CXX,
+            *HOST_FLAGS,
+            "-shared",
+            "-fvisibility=hidden",
+            "-Wno-unused-local-typedefs",
+            "-D__HIP_PLATFORM_AMD__=1",
+            "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *[f"-isystem{p}" for p in cpp_extension.include_paths("cuda")],
+            f"-I{sysconfig.get_paths()['include']}",
+            f"-I{ROOT / 'include'}",
+            str(CSRC / "launch_torch.cpp"),
+            *[f"-L{p}" for p in cpp_extension.library_paths("cuda")],
+            "-ltorch_python",
+            "-ltorch_cpu",
+            "-lc10_hip",
+            "-lc10",
             "-o",
             str(tmp),
         ]

@@ -22,7 +22,7 @@
 struct xt_module {
   std::unique_ptr<xt::Module> ir;
   std::mutex mu;
-  std::map<std::string, xt::Plan> plans;
+  std::map<std::string, std::shared_ptr<const xt::Plan>> plans;
 };
 
 namespace {
@@ -40,21 +40,55 @@ int fail(char** err, int status, const std::string& msg) {
 
 std::string func_key(const char* func) { return func ? std::string(func) : std::string(); }
 
-// Caller holds m->mu.
-int get_plan(xt_module* m, const std::string& func, xt::Plan& out, char** err) {
-  auto it = m->plans.find(func);
+// Caller holds m->mu; the plan stays valid after it is released.  An empty name
+// is the module's only function.
+int get_plan(xt_module* m, const std::string& func, std::shared_ptr<const xt::Plan>& out, char** err) {
+  const std::string& name = func.empty() && m->ir->funcs.size() == 1 ? m->ir->funcs[0].name : func;
+  auto it = m->plans.find(name);
   if (it != m->plans.end()) {
     out = it->second;
     return XT_OK;
   }
-  xt::Plan p;
+  auto p = std::make_shared<xt::Plan>();
   std::string why;
-  if (!xt::build_plan(*m->ir, func, p, why)) return fail(err, XT_ERR_UNSUPPORTED, why);
-  if (p.kind == xt::PlanKind::Fused && !xtk::compile_fused(*p.fused, why))
-    return fail(err, XT_ERR_UNSUPPORTED, "@" + p.func + ": " + why);
-  m->plans.emplace(func, p);
-  out = p;
+  if (!xt::build_plan(*m->ir, name, *p, why)) return fail(err, XT_ERR_UNSUPPORTED, why);
+  if (p->kind == xt::PlanKind::Fused && !xtk::compile_fused(*p->fused, why))
+    return fail(err, XT_ERR_UNSUPPORTED, "@" + p->func + ": " + why);
+  m->plans.emplace(name, p);
+  out = std::move(p);
   return XT_OK;
+}
+
+// Enqueues a plan over buffers known to hold its memrefs.
+int run_plan(const xt::Plan& p, void* const* bufs, void* stream, char** err) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  std::string why;
+  hipError_t e = hipSuccess;
+  switch (p.kind) {
+    case xt::PlanKind::EwBinary: e = xtk::launch_ew_binary(p, bufs, s, why); break;
+    case xt::PlanKind::RowSoftmax: e = xtk::launch_row_softmax(p, bufs, s, why); break;
+    case xt::PlanKind::Gemm: e = xtk::launch_gemm(p, bufs, s, why); break;
+    case xt::PlanKind::Conv2d: e = xtk::launch_conv2d(p, bufs, s, why); break;
+    case xt::PlanKind::TileVM: e = xtk::launch_tilevm(p, bufs, s, why); break;
+    case xt::PlanKind::Fused: e = xtk::launch_fused(p, bufs, s, why); break;
+  }
+  if (!why.empty()) return fail(err, XT_ERR_ARGUMENT, why);
+  if (e != hipSuccess)
+    return fail(err, XT_ERR_DEVICE,
+                std::string("HIP launch failed: ") + hipGetErrorString(e) + " (" + p.describe() +
+                    ")");
+  return XT_OK;
+}
+
+int elem_code(xt::Elem e) {
+  switch (e) {
+    case xt::Elem::F32: return XT_F32;
+    case xt::Elem::F16: return XT_F16;
+    case xt::Elem::BF16: return XT_BF16;
+    case xt::Elem::I8: return XT_I8;
+    case xt::Elem::I32: return XT_I32;
+    default: return -1;
+  }
 }
 
 }  // namespace
@@ -155,12 +189,13 @@ int xt_func_signature(xt_module* m, const char* func, char** out_json, char** er
 int xt_plan(xt_module* m, const char* func, char** out_desc, double* algo_bytes,
             double* algo_flops, char** err) {
   if (!m) return fail(err, XT_ERR_TYPE, "expected an xtile module");
-  xt::Plan p;
+  std::shared_ptr<const xt::Plan> plan;
   {
     std::lock_guard<std::mutex> lock(m->mu);
-    int st = get_plan(m, func_key(func), p, err);
+    int st = get_plan(m, func_key(func), plan, err);
     if (st != XT_OK) return st;
   }
+  const xt::Plan& p = *plan;
   if (out_desc) *out_desc = dup_string(p.describe());
   if (algo_bytes) *algo_bytes = p.algo_bytes;
   if (algo_flops) *algo_flops = p.algo_flops;
@@ -170,12 +205,13 @@ int xt_plan(xt_module* m, const char* func, char** out_desc, double* algo_bytes,
 int xt_gpu_run(xt_module* m, const char* func, void* const* bufs, const size_t* buf_bytes,
                int nbufs, void* stream, char** err) {
   if (!m) return fail(err, XT_ERR_TYPE, "expected an xtile module");
-  xt::Plan p;
+  std::shared_ptr<const xt::Plan> plan;
   {
     std::lock_guard<std::mutex> lock(m->mu);
-    int st = get_plan(m, func_key(func), p, err);
+    int st = get_plan(m, func_key(func), plan, err);
     if (st != XT_OK) return st;
   }
+  const xt::Plan& p = *plan;
   if (nbufs != static_cast<int>(p.arg_types.size()))
     return fail(err, XT_ERR_ARGUMENT,
                 "@" + p.func + " takes " + std::to_string(p.arg_types.size()) +
@@ -190,23 +226,32 @@ int xt_gpu_run(xt_module* m, const char* func, void* const* bufs, const size_t* 
                   "buffer " + std::to_string(k) + " holds " + std::to_string(buf_bytes[k]) +
                       " bytes; " + t.str() + " needs " + std::to_string(need));
   }
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  std::string why;
-  hipError_t e = hipSuccess;
-  switch (p.kind) {
-    case xt::PlanKind::EwBinary: e = xtk::launch_ew_binary(p, bufs, s, why); break;
-    case xt::PlanKind::RowSoftmax: e = xtk::launch_row_softmax(p, bufs, s, why); break;
-    case xt::PlanKind::Gemm: e = xtk::launch_gemm(p, bufs, s, why); break;
-    case xt::PlanKind::Conv2d: e = xtk::launch_conv2d(p, bufs, s, why); break;
-    case xt::PlanKind::TileVM: e = xtk::launch_tilevm(p, bufs, s, why); break;
-    case xt::PlanKind::Fused: e = xtk::launch_fused(p, bufs, s, why); break;
+  return run_plan(p, bufs, stream, err);
+}
+
+int xt_gpu_run_buffers(xt_module* m, const char* func, const xt_buffer* bufs, int nbufs, void* stream, char** err) {
+  if (!m) return fail(err, XT_ERR_TYPE, "expected an xtile module");
+  std::shared_ptr<const xt::Plan> plan;
+  {
+    std::lock_guard<std::mutex> lock(m->mu);
+    int st = get_plan(m, func_key(func), plan, err);
+    if (st != XT_OK) return st;
   }
-  if (!why.empty()) return fail(err, XT_ERR_ARGUMENT, why);
-  if (e != hipSuccess)
-    return fail(err, XT_ERR_DEVICE,
-                std::string("HIP launch failed: ") + hipGetErrorString(e) + " (" + p.describe() +
-                    ")");
-  return XT_OK;
+  const xt::Plan& p = *plan;
+  constexpr int kMost = 16;
+  if (nbufs != static_cast<int>(p.arg_types.size()) || nbufs > kMost || !bufs)
+    return fail(err, XT_ERR_ARGUMENT, "@" + p.func + " takes " + std::to_string(p.arg_types.size()) +
+                                          " buffers (at most " + std::to_string(kMost) + " described ones)");
+  void* ptrs[kMost] = {};
+  for (int k = 0; k < nbufs; ++k) {
+    const xt::Type& t = p.arg_types[k];
+    bool same = bufs[k].ptr && bufs[k].dtype == elem_code(t.elem) && bufs[k].rank == static_cast<int>(t.shape.size()) &&
+                (bufs[k].shape || bufs[k].rank == 0);
+    for (int d = 0; same && d < bufs[k].rank; ++d) same = bufs[k].shape[d] == t.shape[d];
+    if (!same) return fail(err, XT_ERR_ARGUMENT, "buffer " + std::to_string(k) + " is not a " + t.str());
+    ptrs[k] = bufs[k].ptr;
+  }
+  return run_plan(p, ptrs, stream, err);
 }
 
 }  // extern "C"
