@@ -30,7 +30,10 @@ const char* kOptions[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang
 
 std::mutex g_mu;
 std::map<std::string, std::string> g_code;                          // source -> code object
-std::map<std::pair<uint64_t, int>, hipFunction_t> g_func;           // (source hash, device) -> kernel
+struct Loaded {
+  hipFunction_t fused = nullptr, attend = nullptr;  // attend: of programs that hold one
+};
+std::map<std::pair<uint64_t, int>, Loaded> g_func;                  // (source hash, device) -> kernels
 
 uint64_t fnv1a(const std::string& s, uint64_t h = 1469598103934665603ull) {
   for (unsigned char c : s) h = (h ^ c) * 1099511628211ull;
@@ -173,7 +176,9 @@ hipError_t launch_fused(const xt::Plan& p, void* const* bufs, hipStream_t s, std
   // the program's scalar-access variant (vw = 1), or the interpreter when
   // that variant does not fit the fused layout.
   uintptr_t align = 0;
-  int bad = misaligned(vm, bufs, fp->vw, align);
+  bool attend = fp->attend_workgroups > 0;
+  for (const xt::VmAccess& a : vm.access) attend = attend && reinterpret_cast<uintptr_t>(bufs[a.arg]) % 16 == 0;
+  int bad = attend ? -1 : misaligned(vm, bufs, fp->vw, align);
   if (bad >= 0 && fp->vw > 1) {
     std::string err;
     const xt::FusedPlan* sp = scalar_variant(p, err);
@@ -211,12 +216,13 @@ hipError_t launch_fused(const xt::Plan& p, void* const* bufs, hipStream_t s, std
       hipModule_t mod = nullptr;
       e = hipModuleLoadData(&mod, fp->code.data());
       if (e != hipSuccess) return e;
-      e = hipModuleGetFunction(&fn, mod, "xt_fused");
+      Loaded l;
+      e = hipModuleGetFunction(&l.fused, mod, "xt_fused");
+      if (e == hipSuccess && fp->attend_workgroups > 0) e = hipModuleGetFunction(&l.attend, mod, "xt_attend");
       if (e != hipSuccess) return e;
-      g_func.emplace(key, fn);  // the module stays loaded until the process ends
-    } else {
-      fn = it->second;
+      it = g_func.emplace(key, l).first;  // the module stays loaded until the process ends
     }
+    fn = attend ? it->second.attend : it->second.fused;
   }
   struct {
     void* p[8];
@@ -227,6 +233,9 @@ hipError_t launch_fused(const xt::Plan& p, void* const* bufs, hipStream_t s, std
     why = "fused kernel launch size out of range";
     return hipErrorInvalidValue;
   }
+  if (attend)  // attend_vm checked its grid
+    return hipModuleLaunchKernel(fn, static_cast<unsigned>(fp->attend_workgroups), 1, 1,
+                                 static_cast<unsigned>(fp->attend_threads), 1, 1, 0, s, params, nullptr);
   return hipModuleLaunchKernel(fn, static_cast<unsigned>(fp->workgroups), 1, 1, static_cast<unsigned>(fp->threads), 1, 1, 0,
                                s, params, nullptr);
 }

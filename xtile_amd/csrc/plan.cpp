@@ -1075,6 +1075,7 @@ bool build_plan(const Module& m, const std::string& func, Plan& p, std::string& 
         p.gemm_ftoi = q.gemm_ftoi;
         p.gemm_ragged = true;
       }
+      if (fp.staged) attend_vm(p.vm, p.grid, fp);
       p.kind = PlanKind::Fused;
       p.fused = std::make_shared<FusedPlan>(std::move(fp));
       p.vm_fallback = vm_fits_interpreter(p.vm, p.vm_fallback_why);

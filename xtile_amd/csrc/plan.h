@@ -108,6 +108,9 @@ struct FusedPlan {
   // the first launch whose buffers are not aligned to the vw-element vectors
   std::shared_ptr<FusedPlan> scalar;
   bool staged = false;       // written by stage_vm (values in LDS), not fuse_vm
+  // a staged program whose source also holds attend_vm's kernel `xt_attend`,
+  // which runs when every buffer is 16-byte aligned (0 workgroups: none)
+  int attend_threads = 0, attend_workgroups = 0;
 };
 
 struct Plan {
@@ -159,6 +162,10 @@ bool fuse_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& out, std::strin
 // (LDS beyond 160 KB, more than 8 accesses, an exact matmul of values that
 // are not i8 tiles, a load of a memref the program stored to).
 bool stage_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& out, std::string& why, int max_vw = 4);
+
+// Adds the attention kernel to a staged program of that form (attention.cpp);
+// false, with `fp` as it was, for any other.
+bool attend_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& fp);
 
 // Whether the C tiles of a Gemm plan's Blocks form one [M][N] region at c0 with
 // pitch ld: along one grid axis the Blocks step A and C by a tile's rows (B and

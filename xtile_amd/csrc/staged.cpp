@@ -49,6 +49,9 @@
 //   * the source of a copying permute: an odd pitch (a column read is
 //     conflict-free).
 // The first consumer in program order decides.
+//
+// Attention programs carry a second kernel beside this one (attention.cpp), which
+// runs when the buffers are 16-byte aligned.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
