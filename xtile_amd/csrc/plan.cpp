@@ -394,9 +394,8 @@ bool match_softmax(const Analysis& an, Plan& p, std::string& err) {
   // other shapes and types run on the tile interpreter
   if (t.elem != Elem::F32 || t.rank() != 2 || t.shape[1] > 8192) return false;
   if (!access_of(an, *ld, p.a, err) || !access_of(an, *st, p.c, err)) return false;
-  // rows above 2048 floats are held as float4 vectors: columns, pitches and
-  // tile origins must be multiples of 4 (the buffers' 16-byte alignment is
-  // checked at launch)
+  // rows above 2048 floats run here when columns, pitches and tile origins are
+  // multiples of 4; the fused kernel holds the others in registers too
   auto vec4 = [](const Access2D& a) {
     return a.cols % 4 == 0 && a.ld % 4 == 0 && a.addr.c0 % 4 == 0 && a.addr.sx % 4 == 0 && a.addr.sy % 4 == 0 &&
            a.addr.sz % 4 == 0;
@@ -1031,20 +1030,7 @@ bool build_plan(const Module& m, const std::string& func, Plan& p, std::string& 
   std::string first;
   for (auto match : {match_ew, match_softmax, match_gemm, match_conv}) {
     std::string why;
-    if (match(an, p, why)) {
-      if (p.kind == PlanKind::RowSoftmax) {
-        // the interpreter lowering, for buffers the softmax kernel cannot vectorise
-        Plan q = p;
-        std::string e2;
-        if (match_vm(an, q, e2) && vm_fits_interpreter(q.vm, e2)) {
-          p.vm = std::move(q.vm);
-          p.vm_fallback = true;
-        } else {
-          p.vm_fallback_why = e2.empty() ? "no interpreter lowering" : e2;
-        }
-      }
-      return true;
-    }
+    if (match(an, p, why)) return true;
     if (first.empty()) first = why;
   }
   if (match_vm(an, p, err)) {
