@@ -1,0 +1,60 @@
+"""GPU parity of the small-tile implicit GEMM (kernels/conv_tiles.hip) where its
+tiles, stages and taps do not line up: pixels past the last tile, K ending inside
+a stage, taps of three or five 16-byte chunks, windows outside the image, few and
+many output channels; and of conv_igemm.hip on the same layers
+(XTILE_AMD_CONV_IGEMM=1), which no longer takes them by itself.
+
+f16 / bf16 against the oracle within 4 sqrt(K) 2^-24 (K f32 additions of random
+sign, each rounding by at most 2^-24 of its partial sum); i8 exact."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import xtile_amd as xt
+from oracle import f32_to_bf16_bits
+from tests.conftest import oracle_threads
+from tests.gpu_util import frob_rel, run_gpu, run_oracle
+from xtile_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+_XT = {"f16": xt.float16, "bf16": xt.bfloat16, "i8": xt.int8}
+
+
+@pytest.mark.parametrize("kernel", ["tiles", "igemm"])
+@pytest.mark.parametrize(
+    "n,h,w,cin,cout,kh,kw,pad,stride,dil,dt",
+    [(1, 1, 1, 512, 8, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "f16"),        # one pixel, one stage of 8 channels
+     (1, 5, 7, 264, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "bf16"),      # taps of 33 chunks
+     (3, 9, 9, 24, 200, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16"),       # taps of 3 chunks, channels past 192
+     (2, 13, 11, 40, 256, 5, 3, (0, 1, 3, 2), (2, 1), (1, 2), "bf16"),    # taps of 5, uneven pads, strides, dilations
+     (1, 33, 31, 136, 72, 3, 3, (1, 1, 1, 1), (2, 2), (2, 2), "f16"),     # windows half outside
+     (1, 20, 20, 48, 48, 7, 7, (3, 3, 3, 3), (1, 1), (1, 1), "i8"),       # taps of 3 chunks of bytes
+     (5, 18, 18, 512, 32, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1), "i8"),
+     (2, 7, 7, 96, 528, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),
+     (9, 23, 23, 48, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16")],     # 64 x 64 tiles
+)
+def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt):
+    monkeypatch.setenv("XTILE_AMD_CONV_IMAGE", "0")
+    if kernel == "igemm":
+        monkeypatch.setenv("XTILE_AMD_CONV_IGEMM", "1")
+    oh = (h + pad[0] + pad[2] - dil[0] * (kh - 1) - 1) // stride[0] + 1
+    ow = (w + pad[1] + pad[3] - dil[1] * (kw - 1) - 1) // stride[1] + 1
+    mod = K.conv2d(n, h, w, cin, cout, kh, kw, 1, ow, dtype=_XT[dt], pad=pad, stride=stride, dilation=dil)
+    rng = np.random.default_rng(h * cin)
+    if dt == "i8":
+        x = rng.integers(-128, 128, (n, h, w, cin), dtype=np.int8)
+        f = rng.integers(-128, 128, (kh, kw, cin, cout), dtype=np.int8)
+    else:
+        x = rng.normal(0, 0.1, (n, h, w, cin)).astype(np.float32)
+        f = rng.normal(0, 0.1, (kh, kw, cin, cout)).astype(np.float32)
+        x, f = (x.astype(np.float16), f.astype(np.float16)) if dt == "f16" else (f32_to_bf16_bits(x), f32_to_bf16_bits(f))
+    bufs = [x, f, np.full((n, oh, ow, cout), np.nan, np.float32)]
+    got = run_gpu(mod, bufs, [dt, dt, "f32"], cuda, case=f"conv {kernel} {n}x{h}x{w}x{cin}->{cout} {kh}x{kw} {dt}")[2]
+    want = run_oracle(mod, bufs, oracle_threads())[2]
+    if dt == "i8":
+        assert np.array_equal(got, want)
+    else:
+        assert frob_rel(got, want) <= 4 * np.sqrt(kh * kw * cin) * 2.0**-24

@@ -57,6 +57,7 @@
 //     band kernel: this one re-reads every input pixel once per tap from L2
 //     and took 17.3 us there against 13.0.
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 #include "launch.h"
@@ -525,6 +526,26 @@ bool conv_blocks_cover_output(const xt::Plan& p, long long es) {
   return !(c.filt_addr.sx || c.filt_addr.sy || c.filt_addr.sz || (c.filt_addr.c0 * es) % 16);
 }
 
+// Estimated microseconds of this file's kernel and of conv_tiles.hip's on one
+// layer, fitted to graph-replay times of 40 layers from 32 pixels x 16 channels
+// to 124509 x 16.  Here a stage took 0.44 us (0.36 with loader waves) whatever
+// the tile while a CU has one workgroup, and a launch 5.2, a K split 2.5 for the
+// zero fill and 2 a million atomic sums; there a round of tiles costs its start
+// and end and its operands at ~70 KB a us.  (Measured / estimated: 5 x 18^2 x 512
+// -> 32 3 x 3 / 2 i8 36.6 / 36.9 here, 7.1 / 7.7 in 32 x 32 tiles; 53 x 47^2 x 40
+// -> 64 5 x 5 / 2 30.6 / 26.5, 15.3 / 14.9 in 64 x 64; 32 x 28^2 x 128 -> 128 20.1
+// / 21.0, 30.8 / 26.9.)
+static double igemm_us(bool deep, int stages, long long nwg, long long ksplit, long long outputs, int cus) {
+  const double load = std::max(1.0, 0.85 * double(nwg) / cus);
+  return 5.2 + (deep ? 0.36 : 0.44) * stages / ksplit * load + (ksplit > 1 ? 2.5 + 2e-6 * outputs * ksplit : 0);
+}
+
+static double conv_tiles_us(int bm, int bn, long long M, long long co, long long kbytes, int cus) {
+  const double start = bm == 64 ? 3.2 : bn == 64 ? 2.1 : 1.5, rate = bm + bn > 64 ? 75 : 65;
+  const double n = double((M + bm - 1) / bm * ((co + bn - 1) / bn)) / cus;
+  return 1.8 + std::max(1.0, std::min(std::ceil(n), n + 0.5)) * (start + double(bm + bn) * kbytes / 1024 / rate);
+}
+
 bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e) {
   const xt::ConvPlan& c = p.conv;
   const bool i8 = c.elem == xt::Elem::I8;
@@ -606,6 +627,20 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   a.kstages = (int)(a.stages / ksplit);
   const long long nwg = tiles * ksplit;
   if (!grid_fits(nwg, 256) || M * c.CO % 4) return false;
+  // Few tiles: conv_tiles.hip's, where they are estimated well ahead
+  // (XTILE_AMD_CONV_IGEMM=1 keeps this kernel).
+  const char* own = std::getenv("XTILE_AMD_CONV_IGEMM");
+  if (!(own && own[0] == '1')) {
+    const double here = igemm_us(deep, a.stages, nwg, ksplit, M * c.CO, cus);
+    const int shapes[3][2] = {{64, 64}, {32, 64}, {32, 32}};
+    int best = -1;
+    double us = 0.85 * here;
+    for (int k = 0; k < 3; ++k) {
+      const double t = conv_tiles_us(shapes[k][0], shapes[k][1], M, c.CO, K * es, cus);
+      if (t < us) us = t, best = k;
+    }
+    if (best >= 0 && run_conv_tiles(p, bufs, gB * c.TB, shapes[best][0], shapes[best][1], s, e)) return true;
+  }
   a.tiles = (int)tiles;
   a.ksplit = (int)ksplit;
   // the rotated walk keeps a whole filter and the XCD's input rows in its

@@ -25,13 +25,7 @@
 // 23+, 1984 x 1408 x 8064 95 against 84; DMA issued between the MFMAs instead
 // of in one burst before them: 10.8 on 1024^3.
 //
-// Stage layout (per wave): A [BM rows][64 B], then B [64 / ES k rows][BN * ES
-// B].  An instruction fills 1 KB, lane L at byte 16 L; the chunk each lane
-// fetches swizzles the tile: A row r keeps its 16-byte chunk c at c ^ ((r >>
-// 2) & 3), so 16 consecutive rows of a fragment read hit 16 bank groups; a B
-// row of 128 B (16-bit, BN = 64) keeps it at c ^ 4 ((k >> 1) & 1), a B row of
-// 64 B of bytes at c ^ 2 ((k >> 2) & 1), so the rows a half-wave's transposing
-// read covers fill 256 B of banks; narrower B rows fill them as they are.
+// Layouts and the loop are in small_tile.h.
 //
 // DMA (LOAD = kDma): buffer_load ... lds, NS - 1 stages ahead.  Rows past M
 // and column chunks past N are clamped to ones that exist (their results are
@@ -43,27 +37,13 @@
 // accesses), kAhead stages held in registers, written to the same LDS layout.
 // A stage that holds K's end or B's last bytes takes each chunk from a load
 // that ends where its elements end, shifted into place, zeros past K.
-#include <type_traits>
-
-#include "gemm_common.h"
 #include "launch.h"
+#include "small_tile.h"
 
 namespace xtk {
 namespace {
 
 enum { kDma = 0, kRegs = 1 };
-
-constexpr int kStageK = 128;  // K bytes per stage: a whole cache line of every A row
-
-template <int BM, int BN>
-struct SmallTile {
-  static constexpr int STAGE = (BM + BN) * kStageK;
-  static constexpr int NS = BM + BN == 128 ? 2 : BM + BN == 96 ? 3 : 4;  // stages of a wave's ring
-  static constexpr int RING = NS * STAGE;
-  static constexpr int LDC = BN + 8;  // floats per row of a partial tile: half-waves, four rows apart, in distinct banks
-  static constexpr int LDS = 4 * RING;
-  static_assert(4 * BM * LDC * 4 <= LDS, "the partial tiles reuse the rings");
-};
 
 // Sixteen bytes at element alignment.
 template <int ES>
@@ -94,19 +74,8 @@ __device__ __forceinline__ uint4v load_part(const unsigned char* q, int n, const
 
 template <int ELEM, bool OUT_I8, int BM, int BN, int LOAD>
 __global__ __launch_bounds__(256, 1) void gemm_small_kernel(GemmArgs p) {
-  typedef SmallTile<BM, BN> T;
-  typedef typename Acc<ELEM>::type acc_t;
-  typedef __attribute__((address_space(3))) unsigned char lds_t;
-  constexpr int ES = ELEM == kI8 ? 1 : 2;
-  constexpr int MI = BM / 32, NJ = BN / 32;
-  constexpr int AB = BM * kStageK;   // A bytes per stage
-  constexpr int BR = BN * ES;        // bytes of a B row
-  constexpr int KR = kStageK / ES;   // B rows per stage
-  constexpr int KSR = 32 / ES;       // B rows per MFMA step
-  constexpr int STEPS = kStageK / 32;
-  constexpr int PA = BM / 8, PB = BN / 8, PER = PA + PB;
-  constexpr int CPR = BR / 16, RPI = 1024 / BR;
-  constexpr int NS = T::NS;
+  typedef SmallTile<ELEM, BM, BN> T;
+  constexpr int ES = T::ES, AB = T::AB, BR = T::BR, KR = T::KR, PA = T::PA, PB = T::PB, PER = T::PER, RPI = T::RPI;
   __shared__ __attribute__((aligned(1024))) unsigned char lds[T::LDS];
 
   int tx, ty;
@@ -117,75 +86,15 @@ __global__ __launch_bounds__(256, 1) void gemm_small_kernel(GemmArgs p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned char* const ring = lds + wave * T::RING;
 
-  auto bsw = [](int k) { return BR == 128 ? 4 * ((k >> 1) & 1) : ES == 1 && BR == 64 ? 2 * ((k >> 2) & 1) : 0; };
-  // what this lane fetches: A row 8 i + arow, chunk ach(i); B row RPI i + brow, chunk bch
-  const int arow = lane >> 3;
-  auto ach = [&](int i) { return (lane & 7) ^ ((4 * i + (lane >> 4)) & 7); };
-  const int brow = lane / CPR;
-  int bch = (lane % CPR) ^ bsw(brow);
+  const int arow = lane >> 3, brow = lane / T::CPR;
+  auto ach = [&](int i) { return T::a_chunk(lane, i); };
+  int bch = T::b_chunk(lane);
   if (bch * (16 / ES) >= nleft) bch = 0;
   const int ns = (p.K * ES + kStageK - 1) / kStageK;  // stages; this wave's: wave, wave + 4, ...
   const int mine = (ns - wave + 3) >> 2;
 
-  acc_t acc[MI][NJ];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-
-  const int lrow = lane & 31, hi = lane >> 5;
-  int aoff[MI], asw[MI], boff[NJ][2];
-#pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int r = i * 32 + lrow;
-    aoff[i] = r * kStageK;
-    asw[i] = (r >> 1) & 7;
-  }
-  {
-    const int g = lane >> 4, li = lane & 15;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int k = ES == 2 ? 8 * (g >> 1) + 4 * h + (li >> 2) : 16 * (g >> 1) + 8 * h + (li >> 1);
-        const int cb = ES == 2 ? (j * 32 + 16 * (g & 1) + 4 * (li & 3)) * 2 : j * 32 + 16 * (g & 1) + 8 * (li & 1);
-        boff[j][h] = AB + k * BR + (((cb >> 4) ^ bsw(k)) << 4) + (cb & 15);
-      }
-  }
-  // the fragments of a stage
-  uint4v af[STEPS][MI], bf[STEPS][NJ];
-  auto read_stage = [&](const unsigned char* S) {
-#pragma unroll
-    for (int ks = 0; ks < STEPS; ++ks) {
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-        af[ks][i] = *reinterpret_cast<const uint4v*>(S + aoff[i] + (((ks * 2 + hi) ^ asw[i]) << 4));
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        lds_t* const f = (lds_t*)(S + ks * KSR * BR);
-        uint2v lo, up;
-        if constexpr (ES == 2) {
-          lo = __builtin_bit_cast(uint2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                              reinterpret_cast<short4v __attribute__((address_space(3)))*>(f + boff[j][0])));
-          up = __builtin_bit_cast(uint2v, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                              reinterpret_cast<short4v __attribute__((address_space(3)))*>(f + boff[j][1])));
-        } else {
-          lo = __builtin_bit_cast(uint2v, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                                              reinterpret_cast<int2v __attribute__((address_space(3)))*>(f + boff[j][0])));
-          up = __builtin_bit_cast(uint2v, __builtin_amdgcn_ds_read_tr8_b64_v2i32(
-                                              reinterpret_cast<int2v __attribute__((address_space(3)))*>(f + boff[j][1])));
-        }
-        bf[ks][j] = uint4v{lo[0], lo[1], up[0], up[1]};
-      }
-    }
-  };
-  // MFMA n of a stage's STEPS MI NJ
-  auto mma = [&](int n) {
-    const int ks = n / (MI * NJ), i = n / NJ % MI, j = n % NJ;
-    acc[i][j] = mfma<ELEM>(af[ks][i], bf[ks][j], acc[i][j]);
-  };
+  T t4;
+  t4.begin(lane);
 
   if constexpr (LOAD == kDma) {
     // K past the end: offsets at 2^31, past the records of a descriptor that
@@ -197,51 +106,18 @@ __global__ __launch_bounds__(256, 1) void gemm_small_kernel(GemmArgs p) {
 #pragma unroll
     for (int i = 0; i < PA; ++i) va[i] = (unsigned)min(8 * i + arow, mleft - 1) * lda + (unsigned)ach(i) * 16;
     const unsigned vb = (unsigned)brow * ldb + (unsigned)bch * 16;
-    const unsigned ring_at = lds_addr(ring);
-    // instruction i of wave-stage q (stage 4 q + wave) into ring slot `slot`
-    auto issue = [&](int q, int slot, int i) {
-      const int s = 4 * q + wave;
-      const unsigned at = ring_at + slot * T::STAGE;
+    t4.run(ring, mine, [&](int q, unsigned at, int i) {
+      const int s = __builtin_amdgcn_readfirstlane(4 * q + wave);
       const bool last = tail && s + 1 == ns;
       if (i < PA) {
         const bool in = !last || ach(i) * 16 < p.K * ES - s * kStageK;
-        dma16(ra, at + i * 1024, in ? va[i] : 0x80000000u, (unsigned)s * kStageK);
+        dma16(ra, at + i * 1024, in ? va[i] : 0x80000000u, __builtin_amdgcn_readfirstlane((unsigned)s * kStageK));
       } else {
         const int k = s * KR + RPI * (i - PA);
         const bool in = !last || k + brow < p.K;
-        dma16(rb, at + AB + (i - PA) * 1024, in ? vb : 0x80000000u, (unsigned)k * ldb);
+        dma16(rb, at + AB + (i - PA) * 1024, in ? vb : 0x80000000u, __builtin_amdgcn_readfirstlane((unsigned)k * ldb));
       }
-    };
-    // this wave's stage has landed when at most `ahead` later ones are outstanding
-    auto landed = [&](int ahead) {
-      switch (ahead) {
-        case 0: XTK_WAIT_VM(0); break;
-        case 1: XTK_WAIT_VM(PER); break;
-        case 2: XTK_WAIT_VM(2 * PER); break;
-        default: XTK_WAIT_VM(3 * PER); break;
-      }
-      asm volatile("" ::: "memory");
-    };
-    static_assert((NS - 1) * PER < 64 && NS <= 4, "vmcnt is six bits");
-#pragma unroll
-    for (int q = 0; q < NS; ++q)
-      if (q < mine)
-#pragma unroll
-        for (int i = 0; i < PER; ++i) issue(q, q, i);
-    int slot = 0;
-    for (int q = 0; q < mine; ++q) {
-      landed(min(mine - 1 - q, NS - 1));
-      read_stage(ring + slot * T::STAGE);
-      // every fragment is in registers before the DMA that reuses the slot
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      if (q + NS < mine)
-#pragma unroll
-        for (int i = 0; i < PER; ++i) issue(q + NS, slot, i);
-#pragma unroll
-      for (int n = 0; n < STEPS * MI * NJ; ++n) mma(n);
-      slot = slot + 1 == NS ? 0 : slot + 1;
-    }
+    });
   } else {
     constexpr int kAhead = 2;
     uint4v reg[kAhead][PER];
@@ -282,42 +158,22 @@ __global__ __launch_bounds__(256, 1) void gemm_small_kernel(GemmArgs p) {
 #pragma unroll
         for (int i = 0; i < PER; ++i) *reinterpret_cast<uint4v*>(S + i * 1024 + lane * 16) = reg[u][i];
         if (q + kAhead < mine) fetch(q + kAhead, reg[u]);
-        read_stage(S);
-#pragma unroll
-        for (int n = 0; n < STEPS * MI * NJ; ++n) mma(n);
+        t4.read_stage(S);
+        t4.multiply();
       }
   }
 
-  // the four partial tiles through LDS: accumulator register v of tile (i, j)
-  // holds row 8 (v / 4) + 4 hi + v % 4, column lane % 32
-  __syncthreads();
-  typedef typename std::conditional<ELEM == kI8, int, float>::type num_t;
-  num_t* const part = reinterpret_cast<num_t*>(lds);
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v)
-        part[(wave * BM + i * 32 + (v >> 2) * 8 + hi * 4 + (v & 3)) * T::LDC + j * 32 + lrow] = acc[i][j][v];
-  __syncthreads();
   const bool hs = p.has_scale, hb = p.has_bias;
-  constexpr int TPR = BN / 4;  // threads per output row, four columns each
-  const int n0 = 4 * (tid % TPR);
   float sv[4] = {1.f, 1.f, 1.f, 1.f}, bv[4] = {0.f, 0.f, 0.f, 0.f};
+  const int col = 4 * (tid % (BN / 4));  // this thread's output columns
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (n0 + e < nleft) {
-      if (hs) sv[e] = t.S[n0 + e];
-      if (hb) bv[e] = t.Bias[n0 + e];
+    if (col + e < nleft) {
+      if (hs) sv[e] = t.S[col + e];
+      if (hb) bv[e] = t.Bias[col + e];
     }
-#pragma unroll
-  for (int m = tid / TPR; m < BM; m += 256 / TPR) {
-    typedef num_t num4 __attribute__((ext_vector_type(4)));
-    num4 x = *reinterpret_cast<const num4*>(part + m * T::LDC + n0);
-#pragma unroll
-    for (int w = 1; w < 4; ++w) x += *reinterpret_cast<const num4*>(part + (w * BM + m) * T::LDC + n0);
-    if (m >= mleft || n0 >= nleft) continue;
+  t4.finish(lds, wave, [&](int m, int n0, typename T::num4 x) {
+    if (m >= mleft || n0 >= nleft) return;
     const long long off = t.c_off + (long long)m * p.ldc + n0;
     float y[4];
 #pragma unroll
@@ -345,7 +201,7 @@ __global__ __launch_bounds__(256, 1) void gemm_small_kernel(GemmArgs p) {
           if (n0 + e < nleft) c[e] = y[e];
       }
     }
-  }
+  });
 }
 
 template <int ELEM, bool OUT_I8, int LOAD>

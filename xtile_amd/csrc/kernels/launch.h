@@ -71,6 +71,9 @@ hipError_t launch_conv2d_general(const xt::Plan& p, void* const* bufs, hipStream
 // The implicit-GEMM conv kernel (conv_igemm.hip): false, with nothing
 // launched, when the plan is outside what it takes; else `e` is the launch's status.
 bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e);
+// conv_tiles.hip over a plan that launch_conv2d_igemm takes, in bm x bn tiles
+// (64 x 64, 32 x 64 or 32 x 32): false when they exceed one launch.
+bool run_conv_tiles(const xt::Plan& p, void* const* bufs, long long images, int bm, int bn, hipStream_t s, hipError_t& e);
 // The resident-image conv kernel (conv_image.hip), same contract.
 bool launch_conv2d_image(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e);
 // Whether a conv plan's Blocks tile images [0, grid[batch axis] * TB) x every
