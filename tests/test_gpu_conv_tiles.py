@@ -23,23 +23,7 @@ pytestmark = pytest.mark.gpu
 _XT = {"f16": xt.float16, "bf16": xt.bfloat16, "i8": xt.int8}
 
 
-@pytest.mark.parametrize("kernel", ["tiles", "igemm"])
-@pytest.mark.parametrize(
-    "n,h,w,cin,cout,kh,kw,pad,stride,dil,dt",
-    [(1, 1, 1, 512, 8, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "f16"),        # one pixel, one stage of 8 channels
-     (1, 5, 7, 264, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "bf16"),      # taps of 33 chunks
-     (3, 9, 9, 24, 200, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16"),       # taps of 3 chunks, channels past 192
-     (2, 13, 11, 40, 256, 5, 3, (0, 1, 3, 2), (2, 1), (1, 2), "bf16"),    # taps of 5, uneven pads, strides, dilations
-     (1, 33, 31, 136, 72, 3, 3, (1, 1, 1, 1), (2, 2), (2, 2), "f16"),     # windows half outside
-     (1, 20, 20, 48, 48, 7, 7, (3, 3, 3, 3), (1, 1), (1, 1), "i8"),       # taps of 3 chunks of bytes
-     (5, 18, 18, 512, 32, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1), "i8"),
-     (2, 7, 7, 96, 528, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),
-     (9, 23, 23, 48, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16")],     # 64 x 64 tiles
-)
-def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt):
-    monkeypatch.setenv("XTILE_AMD_CONV_IMAGE", "0")
-    if kernel == "igemm":
-        monkeypatch.setenv("XTILE_AMD_CONV_IGEMM", "1")
+def _conv(cuda, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt, kernel):
     oh = (h + pad[0] + pad[2] - dil[0] * (kh - 1) - 1) // stride[0] + 1
     ow = (w + pad[1] + pad[3] - dil[1] * (kw - 1) - 1) // stride[1] + 1
     mod = K.conv2d(n, h, w, cin, cout, kh, kw, 1, ow, dtype=_XT[dt], pad=pad, stride=stride, dilation=dil)
@@ -58,3 +42,37 @@ def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, 
         assert np.array_equal(got, want)
     else:
         assert frob_rel(got, want) <= 4 * np.sqrt(kh * kw * cin) * 2.0**-24
+
+
+@pytest.mark.parametrize("kernel", ["tiles", "igemm"])
+@pytest.mark.parametrize(
+    "n,h,w,cin,cout,kh,kw,pad,stride,dil,dt",
+    [(1, 1, 1, 512, 8, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "f16"),        # one pixel, one stage of 8 channels
+     (1, 5, 7, 264, 40, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "bf16"),      # taps of 33 chunks
+     (3, 9, 9, 24, 200, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16"),       # taps of 3 chunks, channels past 192
+     (2, 13, 11, 40, 256, 5, 3, (0, 1, 3, 2), (2, 1), (1, 2), "bf16"),    # taps of 5, uneven pads, strides, dilations
+     (1, 33, 31, 136, 72, 3, 3, (1, 1, 1, 1), (2, 2), (2, 2), "f16"),     # windows half outside
+     (1, 20, 20, 48, 48, 7, 7, (3, 3, 3, 3), (1, 1), (1, 1), "i8"),       # taps of 3 chunks of bytes
+     (5, 18, 18, 512, 32, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1), "i8"),
+     (2, 7, 7, 96, 528, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),
+     (9, 23, 23, 48, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16")],     # 64 x 64 tiles
+)
+def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt):
+    monkeypatch.setenv("XTILE_AMD_CONV_IMAGE", "0")
+    if kernel == "igemm":
+        monkeypatch.setenv("XTILE_AMD_CONV_IGEMM", "1")
+    _conv(cuda, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt, kernel)
+
+
+@pytest.mark.parametrize(
+    "n,h,cin,cout,k,pad,stride,dt",
+    [(20, 28, 128, 128, 3, 1, 1, "f16"),   # 128 x 128 tiles, loader waves, two stages a tap
+     (17, 37, 136, 96, 3, 1, 1, "bf16"),   # 128 x 128, channels past Cout, stages past a tap's channels
+     (13, 47, 96, 64, 5, 2, 2, "f16"),     # 128 x 64, pixels past the last tile
+     (32, 28, 128, 128, 3, 1, 1, "i8"),    # i8 whose filter leaves bands of one row: 128 x 128
+     (26, 28, 192, 72, 5, 2, 1, "i8")],    # 128 x 64 in two channel tiles, the second 8 wide
+)
+def test_conv_loader_waves(cuda, monkeypatch, n, h, cin, cout, k, pad, stride, dt):
+    """conv_igemm.hip's 128 x 128 and 128 x 64 tiles with loader waves."""
+    monkeypatch.setenv("XTILE_AMD_CONV_IGEMM", "1")
+    _conv(cuda, n, h, h, cin, cout, k, k, (pad,) * 4, (stride, stride), (1, 1), dt, "loader waves")

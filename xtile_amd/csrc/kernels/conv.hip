@@ -786,7 +786,9 @@ int ilog2(unsigned v) {
 // rows and columns exactly once, in the output's natural NHWC addressing, and
 // every Block uses one filter.  Returns false (nothing launched) when
 // it does not apply; `e` carries a launch error otherwise.
-bool try_band(const xt::Plan& p, void* const* bufs, hipStream_t s, int max_lds, int cus, hipError_t& e) {
+// `thin`: also bands that the filter leaves LDS for at most half the rows of an
+// even split, of less than half the filter's bytes.
+bool try_band(const xt::Plan& p, void* const* bufs, hipStream_t s, int max_lds, int cus, bool thin, hipError_t& e) {
   const xt::ConvPlan& c = p.conv;
   if (c.cb.axis < 0 || c.ch.axis < 0 || c.cw.axis < 0 || c.cb.axis == c.ch.axis || c.cb.axis == c.cw.axis ||
       c.ch.axis == c.cw.axis)
@@ -837,7 +839,8 @@ bool try_band(const xt::Plan& p, void* const* bufs, hipStream_t s, int max_lds, 
   const long long ipr = (rf_w + ppi - 1) / ppi;
   // rows per band: spread gB * OH rows over the CUs, shrink until LDS fits
   const long long total_rows = gB * c.out_H;
-  long long R = std::min<long long>(c.out_H, (total_rows + cus - 1) / std::max(cus, 1));
+  const long long even = std::min<long long>(c.out_H, (total_rows + cus - 1) / std::max(cus, 1));
+  long long R = even;
   size_t lds = 0;
   long long hrows_max = 0;
   for (; R >= 1; --R) {
@@ -848,7 +851,7 @@ bool try_band(const xt::Plan& p, void* const* bufs, hipStream_t s, int max_lds, 
       break;
     }
   }
-  if (R < 1) return false;
+  if (R < 1 || (!thin && R * 2 <= even && filt_bytes > 2 * hrows_max * rpitch)) return false;
   // the kernel divides pixel indices below 2^16 by multiply-high reciprocals
   if (hrows_max * ipr >= 65536 || R * c.out_W >= 65536 || rf_w >= 65536 || c.out_W >= 65536) return false;
   if (R * c.out_W * c.CO * 4 >= (1LL << 31)) return false;
@@ -985,11 +988,17 @@ hipError_t launch_conv2d(const xt::Plan& p, void* const* bufs, hipStream_t s, st
   const char* igemm_env = std::getenv("XTILE_AMD_CONV_IGEMM");
   const bool igemm_first = igemm_env && igemm_env[0] == '1';
   if (igemm_first && launch_conv2d_igemm(p, bufs, s, e)) return e;
-  if (try_band(p, bufs, s, max_lds, cus, e)) return e;
+  // Bands cut to half the rows of an even split or fewer, whose loads are mostly
+  // the filter's, come behind the implicit GEMM, which takes nearly every plan
+  // that bands do (32 x 28^2 x 128 -> 128 i8, a 147 KB filter, bands of one row
+  // for four: 16.2 us against 10.2; 64 x 112^2 x 32 -> 128 / 2 f16, a 73 KB
+  // filter, bands of four rows and 81 KB for fourteen: 37.4 against 42.5).
+  if (try_band(p, bufs, s, max_lds, cus, false, e)) return e;
   // filters beyond the band kernel's LDS: each image resident in LDS when
   // its channels fit there, else the implicit GEMM with DMA operands
   if (launch_conv2d_image(p, bufs, s, e)) return e;
   if (launch_conv2d_igemm(p, bufs, s, e)) return e;
+  if (try_band(p, bufs, s, max_lds, cus, true, e)) return e;
   // Cin below 8 (the RGB stem): input rows staged in LDS, K in runs of KW * Cin
   if (launch_conv2d_small(p, bufs, s, e)) return e;
   // the persistent kernel: f16 / bf16 in, f32 out, one image per Block, every

@@ -17,8 +17,18 @@
 // kernels; Blocks are independent (README.md:85-89), so the regrouping is a
 // scheduling choice.
 //
-//   * Workgroup tiles of 128 pixels x 128 channels (Cout a multiple of 128)
-//     or 256 x 64, four waves of 64 x 64 (2 x 2 tiles of
+//   * Workgroup tiles of 128 pixels x 128 or 64 channels with eight loader
+//     waves and 128-byte stages, one a CU, where they are estimated ahead
+//     (igemm_lw_us): long K and up to a few rounds of tiles, which bare tiles
+//     spend waiting for one 64-byte stage after another.  Measured against
+//     those: 32 x 28^2 x 128 -> 128 f16 20.1 -> 12.6 us, 54 x 16^2 x 512 -> 256
+//     57.8 -> 38, 15 x 37^2 x 512 -> 96 61 -> 32, 32 x 28^2 x 192 -> 64 5 x 5 48.6
+//     -> 30 (128 x 64), 32 x 28^2 x 512 -> 512 150 -> 140; but 64 x 56^2 x 64 ->
+//     192 83 against 95 and 1 x 1 layers of few stages, which stay.  (Five
+//     64-byte stages with loader waves 16.4 on the first, four loader waves
+//     14.1, 256 x 64 tiles of three stages behind 128 x 64 or 128 x 128 on
+//     every layer tried; conv_image.hip over bands of rows 15.3-17.3.)
+//   * Else tiles of 128 pixels x 128 channels (Cout a multiple of 128) or 256 x 64, four waves of 64 x 64 (2 x 2 tiles of
 //     v_mfma_f32_32x32x16_{f16,bf16}, f32 sums, or v_mfma_i32_32x32x32_i8,
 //     exact i32 sums rounded to f32 once); 64 or 80 KB of LDS, so two
 //     workgroups share a CU and one's barrier waits are the other's MFMA time.
@@ -540,10 +550,18 @@ static double igemm_us(bool deep, int stages, long long nwg, long long ksplit, l
   return 5.2 + (deep ? 0.36 : 0.44) * stages / ksplit * load + (ksplit > 1 ? 2.5 + 2e-6 * outputs * ksplit : 0);
 }
 
+// Rounds of n CU-fulls of tiles, one a CU: the last one's start overlaps.
+static double tile_rounds(double n) { return std::max(1.0, std::min(std::ceil(n), n + 0.5)); }
+
+// 128 x bn tiles (bn 128 or 64) with loader waves and 128-byte stages, one a CU.
+static double igemm_lw_us(int bn, long long M, long long co, long long stages, int cus) {
+  return 1.8 + tile_rounds(double((M + 127) / 128 * ((co + bn - 1) / bn)) / cus) * (3 + (bn == 128 ? 0.47 : 0.31) * stages);
+}
+
 static double conv_tiles_us(int bm, int bn, long long M, long long co, long long kbytes, int cus) {
   const double start = bm == 64 ? 3.2 : bn == 64 ? 2.1 : 1.5, rate = bm + bn > 64 ? 75 : 65;
   const double n = double((M + bm - 1) / bm * ((co + bn - 1) / bn)) / cus;
-  return 1.8 + std::max(1.0, std::min(std::ceil(n), n + 0.5)) * (start + double(bm + bn) * kbytes / 1024 / rate);
+  return 1.8 + tile_rounds(n) * (start + double(bm + bn) * kbytes / 1024 / rate);
 }
 
 bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e) {
@@ -603,12 +621,16 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   // stages 23.0; 392 tiles of 64 x 64 23.7).
   const bool wide = c.CO % 128 == 0;
   const long long tiles128 = (M + 127) / 128 * ((c.CO + 127) / 128);
-  const bool deep = wide && tiles128 * 2 <= cus && (c.C * es) % 128 == 0;
-  const int bm = deep ? 64 : wide ? 128 : 256, bn = wide ? 128 : 64, kb = deep ? 128 : 64;
-  a.cs = (int)((c.C * es + kb - 1) / kb);
-  a.stages = (int)(c.KH * c.KW) * a.cs;
-  a.ntiles = (int)((c.CO + bn - 1) / bn);
-  const long long tiles = (M + bm - 1) / bm * a.ntiles;
+  bool deep = wide && tiles128 * 2 <= cus && (c.C * es) % 128 == 0;
+  int bm = deep ? 64 : wide ? 128 : 256, bn = wide ? 128 : 64, kb = deep ? 128 : 64;
+  long long tiles = 0;
+  auto lay = [&]() {
+    a.cs = (int)((c.C * es + kb - 1) / kb);
+    a.stages = (int)(c.KH * c.KW) * a.cs;
+    a.ntiles = (int)((c.CO + bn - 1) / bn);
+    tiles = (M + bm - 1) / bm * a.ntiles;
+  };
+  lay();
   // K split when the tiles fill at most half the CUs (f16 / bf16: i8 sums stay
   // exact and whole): up to one workgroup a CU, at least 16 stages each.
   // Measured (batch 32, 3 x 3, 128 x 128 tiles): 7 x 7 x 512 -> 512 (52
@@ -624,23 +646,36 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   // up to one round of tiles with a long K: two halves of >= 64 stages
   // (14 x 14 x 512 -> 512, 196 tiles, 144 stages: 63.7 us whole, 56.9 split)
   else if (split_ok && tiles <= cus && a.stages >= 128) ksplit = 2;
-  a.kstages = (int)(a.stages / ksplit);
-  const long long nwg = tiles * ksplit;
-  if (!grid_fits(nwg, 256) || M * c.CO % 4) return false;
-  // Few tiles: conv_tiles.hip's, where they are estimated well ahead
-  // (XTILE_AMD_CONV_IGEMM=1 keeps this kernel).
+  // 128 x 128 or 128 x 64 tiles with loader waves, where they are estimated
+  // ahead; small layers go to conv_tiles.hip's (XTILE_AMD_CONV_IGEMM=1 keeps
+  // this file's kernel)
+  double us = igemm_us(deep, a.stages, tiles * ksplit, ksplit, M * c.CO, cus);
+  int lw = 0;
+  for (int n : {128, 64}) {
+    const double t = igemm_lw_us(n, M, c.CO, c.KH * c.KW * ((c.C * es + 127) / 128), cus);
+    if (t < 0.95 * us) us = t, lw = n;
+  }
   const char* own = std::getenv("XTILE_AMD_CONV_IGEMM");
   if (!(own && own[0] == '1')) {
-    const double here = igemm_us(deep, a.stages, nwg, ksplit, M * c.CO, cus);
     const int shapes[3][2] = {{64, 64}, {32, 64}, {32, 32}};
     int best = -1;
-    double us = 0.85 * here;
+    us *= 0.9;
     for (int k = 0; k < 3; ++k) {
       const double t = conv_tiles_us(shapes[k][0], shapes[k][1], M, c.CO, K * es, cus);
       if (t < us) us = t, best = k;
     }
-    if (best >= 0 && run_conv_tiles(p, bufs, gB * c.TB, shapes[best][0], shapes[best][1], s, e)) return true;
+    if (M * c.CO % 4 == 0 && best >= 0 &&
+        run_conv_tiles(p, bufs, gB * c.TB, shapes[best][0], shapes[best][1], s, e))
+      return true;
   }
+  if (lw) {
+    deep = false;
+    bm = 128, bn = lw, kb = 128, ksplit = 1;
+    lay();
+  }
+  a.kstages = (int)(a.stages / ksplit);
+  const long long nwg = tiles * ksplit;
+  if (!grid_fits(nwg, lw ? 768 : 256) || M * c.CO % 4) return false;
   a.tiles = (int)tiles;
   a.ksplit = (int)ksplit;
   // the rotated walk keeps a whole filter and the XCD's input rows in its
@@ -658,7 +693,9 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   const int el = i8 ? kIgI8 : c.elem == xt::Elem::BF16 ? kIgBF16 : kIgF16;
 #define XT_IG(E)                                                                                       \
   do {                                                                                                 \
-    if (deep) hipLaunchKernelGGL((conv_igemm_kernel<E, 64, 128, 32, 64, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
+    if (lw == 128) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 128, 64, 64, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
+    else if (lw) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 64, 64, 32, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
+    else if (deep) hipLaunchKernelGGL((conv_igemm_kernel<E, 64, 128, 32, 64, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
     else if (wide) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 128>), dim3(a.nwg), dim3(256), 0, s, a);      \
     else hipLaunchKernelGGL((conv_igemm_kernel<E, 256, 64>), dim3(a.nwg), dim3(256), 0, s, a);                 \
   } while (0)
