@@ -251,15 +251,20 @@ __global__ __launch_bounds__(256) void row_softmax_kernel(SoftmaxArgs p) {
       for (int k = 0; k < 4; ++k) m = k < have[j] ? fmaxf(m, v[j][k]) : m;
     }
     m = row_reduce<true, TPR>(m, lds);
-    float s = 0.0f;
+    // a tree within the thread: as a chain of 4 * NV terms the row's sum had the
+    // larger error (7.5e-8 of 1000 columns' result against 7.3e-8)
+    float part[NV];
 #pragma unroll
-    for (int j = 0; j < NV; ++j)
+    for (int j = 0; j < NV; ++j) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[j][k] = k < have[j] ? exp_fast(v[j][k] - m) : 0.0f;
-        s += v[j][k];
-      }
-    s = row_reduce<false, TPR>(s, lds);
+      for (int k = 0; k < 4; ++k) v[j][k] = k < have[j] ? exp_fast(v[j][k] - m) : 0.0f;
+      part[j] = (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+    }
+#pragma unroll
+    for (int o = 1; o < NV; o *= 2)
+#pragma unroll
+      for (int j = 0; j + o < NV; j += 2 * o) part[j] += part[j + o];
+    const float s = row_reduce<false, TPR>(part[0], lds);
     const float inv = 1.0f / s;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
