@@ -55,7 +55,12 @@ def _conv(cuda, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt, kernel):
      (1, 20, 20, 48, 48, 7, 7, (3, 3, 3, 3), (1, 1), (1, 1), "i8"),       # taps of 3 chunks of bytes
      (5, 18, 18, 512, 32, 3, 3, (1, 1, 1, 1), (2, 2), (1, 1), "i8"),
      (2, 7, 7, 96, 528, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),
-     (9, 23, 23, 48, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16")],     # 64 x 64 tiles
+     (9, 23, 23, 48, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "f16"),      # 64 x 64 tiles
+     (1, 1, 1, 20, 16, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),         # a last chunk of 4 channels of its own
+     (1, 9, 7, 44, 32, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),         # of 12, in 32 x 32 tiles
+     (2, 13, 11, 40, 272, 5, 3, (0, 1, 3, 2), (2, 1), (1, 2), "i8"),      # of 8, uneven pads, strides, dilations
+     (3, 19, 19, 500, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),      # of 4 after several stages
+     (9, 23, 23, 28, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "i8")],
 )
 def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt):
     monkeypatch.setenv("XTILE_AMD_CONV_IMAGE", "0")
@@ -70,7 +75,9 @@ def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, 
      (17, 37, 136, 96, 3, 1, 1, "bf16"),   # 128 x 128, channels past Cout, stages past a tap's channels
      (13, 47, 96, 64, 5, 2, 2, "f16"),     # 128 x 64, pixels past the last tile
      (32, 28, 128, 128, 3, 1, 1, "i8"),    # i8 whose filter leaves bands of one row: 128 x 128
-     (26, 28, 192, 72, 5, 2, 1, "i8")],    # 128 x 64 in two channel tiles, the second 8 wide
+     (26, 28, 192, 80, 5, 2, 1, "i8"),     # 128 x 64 in two channel tiles, the second 16 wide
+     (26, 28, 172, 80, 5, 2, 1, "i8"),     # the same, the last chunk of a tap 12 channels
+     (32, 28, 132, 128, 3, 1, 1, "i8")],   # 128 x 128, of 4 channels
 )
 def test_conv_loader_waves(cuda, monkeypatch, n, h, cin, cout, k, pad, stride, dt):
     """conv_igemm.hip's 128 x 128 and 128 x 64 tiles with loader waves."""

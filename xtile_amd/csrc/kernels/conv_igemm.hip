@@ -151,7 +151,13 @@ __device__ __forceinline__ int ig_bsw(int k) {
 // waves 17.9).  Reading each stage's fragments during the previous stage's
 // MFMAs, or two K groups of 64 x 64 waves that halve the filter-fragment
 // reads, measured slower on top of it.
-template <int ELEM, int BM, int BN, int WTM = 64, int WTN = 64, int KBY = 64, int LW = 0, int NSTAGES = 4>
+//
+// PART (i8 with Cin a multiple of 4 but not of 16): a tap's last 16-byte chunk
+// starts 16 bytes before its last channel's end, so every chunk lies inside its
+// pixel, and the filter rows of the channels it shares with the chunk before
+// read as zeros (whole numbers: a product with zero adds nothing).
+template <int ELEM, int BM, int BN, int WTM = 64, int WTN = 64, int KBY = 64, int LW = 0, bool PART = false,
+          int NSTAGES = 4>
 __global__ __launch_bounds__(64 * (4 + LW), LW == 0 && NSTAGES * KBY * (BM + BN) <= 80 * 1024 ? 2 : 1) void conv_igemm_kernel(IgArgs p) {
   // stages in LDS (64 or 80 KB, two workgroups a CU): five, or a pipeline
   // that also read each stage's fragments during the previous stage's MFMAs
@@ -252,11 +258,10 @@ __global__ __launch_bounds__(64 * (4 + LW), LW == 0 && NSTAGES * KBY * (BM + BN)
   int alim[PA], blim[PB];
 #pragma unroll
   for (int q = 0; q < PA; ++q) alim[q] = p.C - ach[q];
-  {
-    const bool bcol = n0 * ES + (((lane % CPR) ^ ig_bsw<ES, BR>(lane / CPR)) << 4) < p.CO * ES;
+  const bool bcol = n0 * ES + (((lane % CPR) ^ ig_bsw<ES, BR>(lane / CPR)) << 4) < p.CO * ES;
 #pragma unroll
-    for (int q = 0; q < PB; ++q) blim[q] = bcol ? p.C - RPI * (PB * dw + q) - lane / CPR : -(1 << 30);
-  }
+  for (int q = 0; q < PB; ++q) blim[q] = PART || bcol ? p.C - RPI * (PB * dw + q) - lane / CPR : -(1 << 30);
+  const unsigned back = PART ? 16u - (unsigned)(p.C & 15) : 0u;
 
   // DMA state of the next stage to load: its tap (kh, kw), its channel
   // stage lcc within the tap (first channel c0 = lcc KR), the tap's source
@@ -295,12 +300,23 @@ __global__ __launch_bounds__(64 * (4 + LW), LW == 0 && NSTAGES * KBY * (BM + BN)
 #pragma unroll
     for (int q = 0; q < PA; ++q) {
       const bool in = ain[q] & (c0 < alim[q]);
-      dma16(ra, lds_addr(S + (PA * dw + q) * 1024), in ? abase[q] + soff : kIgOutOfRange, 0);
+      const unsigned shift = PART && c0 + 16 > alim[q] ? back : 0u;
+      dma16(ra, lds_addr(S + (PA * dw + q) * 1024), in ? abase[q] + soff - shift : kIgOutOfRange, 0);
     }
     const unsigned sb = (unsigned)(krow + RPI * PB * dw) * ldb;
 #pragma unroll
-    for (int q = 0; q < PB; ++q)
-      dma16(rb, lds_addr(S + AB + (PB * dw + q) * 1024), c0 < blim[q] ? vb : kIgOutOfRange, sb + q * bstep);
+    for (int q = 0; q < PB; ++q) {
+      unsigned char* const at = S + AB + (PB * dw + q) * 1024;
+      if constexpr (PART) {
+        // positions from the last chunk's start on hold the channels `back` before them
+        const int pos = c0 + p.C - blim[q], whole = p.C & ~15, ch = pos < whole ? pos : pos - (int)back;
+        const bool in = (pos < whole) | ((ch >= whole) & (ch < p.C));
+        const unsigned off = sb + q * bstep + vb - (pos < whole ? 0u : back * ldb);
+        dma16(rb, lds_addr(at), bcol & in ? off : kIgOutOfRange, 0);
+      } else {
+        dma16(rb, lds_addr(at), c0 < blim[q] ? vb : kIgOutOfRange, sb + q * bstep);
+      }
+    }
     // the next stage: the next KR channels of this tap, or the next tap
     if (++lst == p.stages) {
       // past the last stage: wrap to the first (only a rotated walk has
@@ -571,8 +587,12 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   const long long es = i8 ? 1 : 2;
   // a K stage is 64 bytes of one tap's channels (the last stage of a tap
   // padded with zeros), read in 16-byte pieces: Cin * esize and Cout * esize
-  // multiples of 16
-  if (c.out_elem != xt::Elem::F32 || c.TC != c.CO || (c.C * es) % 16 || (c.CO * es) % 16) return false;
+  // multiples of 16, or Cin of whole i8 words, at least one piece (PART: 51 x
+  // 31^2 x 40 -> 128 5 x 5 288 us on the generic kernel, 23.9 here; 20 x 112^2 x 40
+  // -> 16 7 x 7 / 2 299, 35.5; 32 x 14^2 x 500 -> 256 993, 19.4)
+  const bool part = i8 && c.C % 16 != 0;
+  if (c.out_elem != xt::Elem::F32 || c.TC != c.CO || (part ? c.C % 4 || c.C < 16 : (c.C * es) % 16) || (c.CO * es) % 16)
+    return false;
   if (!conv_blocks_cover_output(p, es)) return false;
   const long long gB = p.grid[c.cb.axis];
   // the source batch entries the Blocks read: images [0, gB) of an NHWC tensor
@@ -661,7 +681,7 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
     int best = -1;
     us *= 0.9;
     for (int k = 0; k < 3; ++k) {
-      const double t = conv_tiles_us(shapes[k][0], shapes[k][1], M, c.CO, K * es, cus);
+      const double t = conv_tiles_us(shapes[k][0], shapes[k][1], M, c.CO, c.KH * c.KW * ((c.C * es + 15) / 16 * 16), cus);
       if (t < us) us = t, best = k;
     }
     if (M * c.CO % 4 == 0 && best >= 0 &&
@@ -691,17 +711,18 @@ bool launch_conv2d_igemm(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   a.d_ohw = div31((unsigned)(c.out_H * c.out_W));
   a.d_ow = div31((unsigned)c.out_W);
   const int el = i8 ? kIgI8 : c.elem == xt::Elem::BF16 ? kIgBF16 : kIgF16;
-#define XT_IG(E)                                                                                       \
+#define XT_IG(E, P)                                                                                    \
   do {                                                                                                 \
-    if (lw == 128) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 128, 64, 64, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
-    else if (lw) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 64, 64, 32, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
+    if (lw == 128) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 128, 64, 64, 128, 8, P>), dim3(a.nwg), dim3(768), 0, s, a); \
+    else if (lw) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 64, 64, 32, 128, 8, P>), dim3(a.nwg), dim3(768), 0, s, a); \
     else if (deep) hipLaunchKernelGGL((conv_igemm_kernel<E, 64, 128, 32, 64, 128, 8>), dim3(a.nwg), dim3(768), 0, s, a); \
-    else if (wide) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 128>), dim3(a.nwg), dim3(256), 0, s, a);      \
-    else hipLaunchKernelGGL((conv_igemm_kernel<E, 256, 64>), dim3(a.nwg), dim3(256), 0, s, a);                 \
+    else if (wide) hipLaunchKernelGGL((conv_igemm_kernel<E, 128, 128, 64, 64, 64, 0, P>), dim3(a.nwg), dim3(256), 0, s, a); \
+    else hipLaunchKernelGGL((conv_igemm_kernel<E, 256, 64, 64, 64, 64, 0, P>), dim3(a.nwg), dim3(256), 0, s, a); \
   } while (0)
-  if (el == kIgI8) XT_IG(kIgI8);
-  else if (el == kIgBF16) XT_IG(kIgBF16);
-  else XT_IG(kIgF16);
+  if (part) XT_IG(kIgI8, true);
+  else if (el == kIgI8) XT_IG(kIgI8, false);
+  else if (el == kIgBF16) XT_IG(kIgBF16, false);
+  else XT_IG(kIgF16, false);
 #undef XT_IG
   e = hipGetLastError();
   return true;

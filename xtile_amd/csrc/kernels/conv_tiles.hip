@@ -14,6 +14,11 @@
 // tap (zeros outside the image).  Chunks run through the taps without padding,
 // so few channels cost no idle stages.  Sums are in a fixed order and, for i8,
 // exact.
+//
+// PART (i8 with Cin a multiple of 4 but not of 16): a tap's last chunk starts
+// 16 bytes before its last channel's end, so every chunk lies inside its pixel;
+// the filter rows of the channels it shares with the chunk before are zeros
+// (whole numbers: a product with zero adds nothing).
 #include "launch.h"
 #include "small_tile.h"
 
@@ -32,13 +37,13 @@ struct CtArgs {
   int pad_t, pad_l, sh, sw, dh, dw;
   int M;
   int chunks;  // 16-byte chunks of K: KH * KW * cc
-  int cc;      // chunks a tap: C * esize / 16
+  int cc;      // chunks a tap: C * esize / 16, rounded up
   int ntiles;  // channel tiles
   int nwg;
   Div31 d_ohw, d_ow, d_nt, d_cc, d_kw;
 };
 
-template <int ELEM, int BM, int BN>
+template <int ELEM, int BM, int BN, bool PART>
 __global__ __launch_bounds__(256, 1) void conv_tiles_kernel(CtArgs p) {
   typedef SmallTile<ELEM, BM, BN> T;
   constexpr int ES = T::ES, AB = T::AB, KR = T::KR, PA = T::PA, RPI = T::RPI;
@@ -66,7 +71,7 @@ __global__ __launch_bounds__(256, 1) void conv_tiles_kernel(CtArgs p) {
   const unsigned ldb = (unsigned)(p.CO * ES);
   const int brow = lane / T::CPR, bch = T::b_chunk(lane);
   const bool bin = n0 * ES + bch * 16 < p.CO * ES;
-  const unsigned vb = (unsigned)brow * ldb + (unsigned)(n0 * ES) + (unsigned)bch * 16;
+  const unsigned vcol = (unsigned)(n0 * ES) + (unsigned)bch * 16, vb = (unsigned)brow * ldb + vcol;
 
   T t4;
   t4.begin(lane);
@@ -84,14 +89,21 @@ __global__ __launch_bounds__(256, 1) void conv_tiles_kernel(CtArgs p) {
         const int tap = p.d_cc(k), kh = p.d_kw(tap), kw = tap - kh * p.KW;
         dih[e] = k < p.chunks ? kh * p.dh : 1 << 30;  // past K: outside every image
         diw[e] = kw * p.dw;
-        toff[e] = (unsigned)((kh * p.dh * p.W + diw[e]) * p.C * ES + (k - tap * p.cc) * 16);
+        const int c16 = (k - tap * p.cc) * 16;
+        toff[e] = (unsigned)((kh * p.dh * p.W + diw[e]) * p.C * ES + (PART ? min(c16, p.C - 16) : c16));
       }
     if (i < PA) {
       const bool in = ((unsigned)(ih0[i] + dih[i & 1]) < (unsigned)p.H) & ((unsigned)(iw0[i] + diw[i & 1]) < (unsigned)p.W);
       dma16(ra, at + i * 1024, in ? base[i] + toff[i & 1] : kCtOutOfRange, 0);
     } else {
       const int k = s * KR + RPI * (i - PA);
-      dma16(rb, at + AB + (i - PA) * 1024, bin & (k + brow < p.K) ? vb + (unsigned)k * ldb : kCtOutOfRange, 0);
+      if constexpr (PART) {
+        const int chunk = (k + brow) >> 4, tap = p.d_cc(chunk), c16 = (chunk - tap * p.cc) * 16;
+        const int ch = min(c16, p.C - 16) + ((k + brow) & 15);
+        const bool in = bin & (chunk < p.chunks) & (ch >= c16);
+        dma16(rb, at + AB + (i - PA) * 1024, in ? (unsigned)(tap * p.C + ch) * ldb + vcol : kCtOutOfRange, 0);
+      } else
+        dma16(rb, at + AB + (i - PA) * 1024, bin & (k + brow < p.K) ? vb + (unsigned)k * ldb : kCtOutOfRange, 0);
     }
   });
   t4.finish(lds, wave, [&](int m, int n, typename T::num4 x) {
@@ -102,12 +114,12 @@ __global__ __launch_bounds__(256, 1) void conv_tiles_kernel(CtArgs p) {
   });
 }
 
-template <int ELEM>
+template <int ELEM, bool PART = false>
 void launch_tiles(int bm, int bn, const CtArgs& a, hipStream_t s) {
   const dim3 grid(a.nwg), block(256);
-  if (bm == 64) hipLaunchKernelGGL((conv_tiles_kernel<ELEM, 64, 64>), grid, block, 0, s, a);
-  else if (bn == 64) hipLaunchKernelGGL((conv_tiles_kernel<ELEM, 32, 64>), grid, block, 0, s, a);
-  else hipLaunchKernelGGL((conv_tiles_kernel<ELEM, 32, 32>), grid, block, 0, s, a);
+  if (bm == 64) hipLaunchKernelGGL((conv_tiles_kernel<ELEM, 64, 64, PART>), grid, block, 0, s, a);
+  else if (bn == 64) hipLaunchKernelGGL((conv_tiles_kernel<ELEM, 32, 64, PART>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((conv_tiles_kernel<ELEM, 32, 32, PART>), grid, block, 0, s, a);
 }
 
 }  // namespace
@@ -137,8 +149,8 @@ bool run_conv_tiles(const xt::Plan& p, void* const* bufs, long long images, int 
   a.dh = (int)c.dil_h;
   a.dw = (int)c.dil_w;
   a.M = (int)M;
-  a.cc = (int)(c.C * es / 16);
-  a.chunks = (int)(K * es / 16);
+  a.cc = (int)((c.C * es + 15) / 16);
+  a.chunks = (int)(c.KH * c.KW) * a.cc;
   a.ntiles = (int)((c.CO + bn - 1) / bn);
   const long long nwg = (M + bm - 1) / bm * a.ntiles;
   if (!grid_fits(nwg, 256)) return false;
@@ -149,7 +161,7 @@ bool run_conv_tiles(const xt::Plan& p, void* const* bufs, long long images, int 
   a.d_cc = div31((unsigned)a.cc);
   a.d_kw = div31((unsigned)a.KW);
   switch (c.elem) {
-    case xt::Elem::I8: launch_tiles<kI8>(bm, bn, a, s); break;
+    case xt::Elem::I8: c.C % 16 ? launch_tiles<kI8, true>(bm, bn, a, s) : launch_tiles<kI8>(bm, bn, a, s); break;
     case xt::Elem::BF16: launch_tiles<kBF16>(bm, bn, a, s); break;
     default: launch_tiles<kF16>(bm, bn, a, s); break;
   }
