@@ -60,7 +60,8 @@ def _conv(cuda, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt, kernel):
      (1, 9, 7, 44, 32, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),         # of 12, in 32 x 32 tiles
      (2, 13, 11, 40, 272, 5, 3, (0, 1, 3, 2), (2, 1), (1, 2), "i8"),      # of 8, uneven pads, strides, dilations
      (3, 19, 19, 500, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),      # of 4 after several stages
-     (9, 23, 23, 28, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "i8")],
+     (9, 23, 23, 28, 64, 5, 5, (2, 2, 2, 2), (1, 1), (1, 1), "i8"),
+     (19, 112, 112, 20, 16, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8")],   # conv_small.hip's by itself
 )
 def test_conv_tiles(cuda, monkeypatch, kernel, n, h, w, cin, cout, kh, kw, pad, stride, dil, dt):
     monkeypatch.setenv("XTILE_AMD_CONV_IMAGE", "0")

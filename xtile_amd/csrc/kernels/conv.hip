@@ -997,10 +997,11 @@ hipError_t launch_conv2d(const xt::Plan& p, void* const* bufs, hipStream_t s, st
   // filters beyond the band kernel's LDS: each image resident in LDS when
   // its channels fit there, else the implicit GEMM with DMA operands
   if (launch_conv2d_image(p, bufs, s, e)) return e;
+  if (launch_conv2d_small(p, bufs, s, true, e)) return e;
   if (launch_conv2d_igemm(p, bufs, s, e)) return e;
   if (try_band(p, bufs, s, max_lds, cus, true, e)) return e;
   // Cin below 8 (the RGB stem): input rows staged in LDS, K in runs of KW * Cin
-  if (launch_conv2d_small(p, bufs, s, e)) return e;
+  if (launch_conv2d_small(p, bufs, s, false, e)) return e;
   // the persistent kernel: f16 / bf16 in, f32 out, one image per Block, every
   // output channel, 16-byte channel runs; anything else takes the generic kernel
   if (!persistent_ok) return launch_conv2d_general(p, bufs, s, why);

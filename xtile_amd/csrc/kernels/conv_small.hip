@@ -390,9 +390,15 @@ hipError_t launch_sc(bool big, int tasks_npr, long long wgs, size_t lds, hipStre
 
 }  // namespace
 
-bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e) {
+// `ahead`: only the layers where this kernel is the faster of it and the implicit
+// GEMM: 20 bytes of channels, or up to 28 of a 1 x 1 filter, walked as tasks in
+// rows that fill their chunks (32 x 112^2 x 20 -> 64 3 x 3 39.0 us, 47.2 there;
+// 32 x 112^2 x 24 -> 64 1 x 1 20.0, 25.0; but 24 -> 32 3 x 3 44.6 against 39.0 and
+// 64 x 56^2 x 20 -> 64, rows of 56 in chunks of 128, 37.0 against 25.0).
+bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, bool ahead, hipError_t& e) {
   const xt::ConvPlan& c = p.conv;
   const bool i8 = c.elem == xt::Elem::I8;
+  if (ahead && !(i8 && c.C >= 16 && (c.C <= 20 || (c.C <= 28 && c.KH * c.KW == 1)))) return false;
   if (c.elem != xt::Elem::F16 && c.elem != xt::Elem::BF16 && !i8) return false;
   const long long es = i8 ? 1 : 2, ks = i8 ? 32 : 16, fr = 64 * es;
   // 16-byte filter pieces: Cout * esize a multiple of 16
@@ -467,6 +473,7 @@ bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
   const size_t lds_tasks = (size_t)(c.KH * 256 * a.npr * es + kp * fr + kp * 2);
   const bool tasks = ntiles == 1 && a.npr <= 4 && c.KH * a.npr <= 28 && ntask >= 2048 &&
                      c.KH * 256 * a.npr * es < 65536 && 3 * lds_tasks <= size_t(kMaxLds);
+  if (ahead && !(tasks && c.out_W * 8 >= chunks * 128 * 7)) return false;
   if (tasks) {
     int cus = 256, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||

@@ -82,7 +82,7 @@ bool launch_conv2d_image(const xt::Plan& p, void* const* bufs, hipStream_t s, hi
 // element); shared by the implicit-GEMM and resident-image kernels.
 bool conv_blocks_cover_output(const xt::Plan& p, long long es);
 // The few-input-channel conv kernel (conv_small.hip), same contract.
-bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, hipError_t& e);
+bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, bool ahead, hipError_t& e);
 hipError_t launch_tilevm(const xt::Plan& p, void* const* bufs, hipStream_t s, std::string& why);
 
 // Fused tile programs (fused_jit.cpp): compile_fused fills fp.code from
