@@ -391,10 +391,11 @@ hipError_t launch_sc(bool big, int tasks_npr, long long wgs, size_t lds, hipStre
 }  // namespace
 
 // `ahead`: only the layers where this kernel is the faster of it and the implicit
-// GEMM: 20 bytes of channels, or up to 28 of a 1 x 1 filter, walked as tasks in
-// rows that fill their chunks (32 x 112^2 x 20 -> 64 3 x 3 39.0 us, 47.2 there;
-// 32 x 112^2 x 24 -> 64 1 x 1 20.0, 25.0; but 24 -> 32 3 x 3 44.6 against 39.0 and
-// 64 x 56^2 x 20 -> 64, rows of 56 in chunks of 128, 37.0 against 25.0).
+// GEMM: 20 bytes of channels, or up to 28 of a 1 x 1 filter, one channel tile,
+// enough output rows for eight workgroups a CU and rows that fill their chunks
+// (32 x 112^2 x 20 -> 64 3 x 3 39.0 us, 47.2 there; 32 x 112^2 x 24 -> 64 1 x 1
+// 20.0, 25.0; but 24 -> 32 3 x 3 44.6 against 39.0, 64 x 56^2 x 20 -> 64, rows of
+// 56 in chunks of 128, 37.0 against 25.0, and 8 x 112^2 x 20 -> 64 15.3, 13.8).
 bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, bool ahead, hipError_t& e) {
   const xt::ConvPlan& c = p.conv;
   const bool i8 = c.elem == xt::Elem::I8;
@@ -427,6 +428,7 @@ bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, bo
   if (lds > size_t(kMaxLds) || images > c.N) return false;
   const long long chunks = (c.out_W + 127) / 128, ntiles = (c.CO + 63) / 64;
   const long long wgs = images * c.out_H * chunks * ntiles;
+  if (ahead && !(ntiles == 1 && wgs >= 2048 && c.out_W * 8 >= chunks * 128 * 7)) return false;
   const long long src_bytes = images * c.H * c.W * c.C * es, filt_bytes = c.KH * run * c.CO * es;
   if (!grid_fits(wgs, 256) || src_bytes >= (1LL << 31) || filt_bytes >= (1LL << 31)) return false;
   const unsigned char* src = static_cast<const unsigned char*>(bufs[c.src_arg]);
@@ -473,7 +475,6 @@ bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, bo
   const size_t lds_tasks = (size_t)(c.KH * 256 * a.npr * es + kp * fr + kp * 2);
   const bool tasks = ntiles == 1 && a.npr <= 4 && c.KH * a.npr <= 28 && ntask >= 2048 &&
                      c.KH * 256 * a.npr * es < 65536 && 3 * lds_tasks <= size_t(kMaxLds);
-  if (ahead && !(tasks && c.out_W * 8 >= chunks * 128 * 7)) return false;
   if (tasks) {
     int cus = 256, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
