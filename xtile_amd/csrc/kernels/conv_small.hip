@@ -1,6 +1,7 @@
 // xt.load_conv2d with few input channels (Cin * esize not a multiple of 16:
 // the RGB stem of a CNN; any Cin whose row of channels is not a whole number
-// of 16-byte pieces: 3, 5, 12, 20 ... for f16 / bf16, 3, 12, 15 ... for i8) as an
+// of 16-byte pieces: 3, 5, 12, 20 ... for f16 / bf16, 3, 12, 15, 18 ... for i8,
+// whose multiples of 4 from 20 on go to the implicit GEMM where it is faster) as an
 // implicit GEMM over an input patch staged in LDS, for f16 / bf16 / i8 sources
 // and an f32 result.
 //
