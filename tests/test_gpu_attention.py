@@ -144,3 +144,27 @@ def test_buffers_off_the_alignment(cuda, off):
     xt.launch(m, *dev)
     torch.cuda.synchronize()
     assert frob_rel(dev[3].cpu().numpy(), run_oracle(m, bufs, 1)[3]) <= 1e-5
+
+
+@pytest.mark.parametrize("how", ["one memref", "one tensor"])
+def test_result_over_the_values(cuda, how):
+    """The result stored over V, a Block's own tile each: as one memref of the
+    program, and as one tensor passed for both.  Either runs one workgroup a
+    Block, which has V in LDS before it stores."""
+    import torch
+
+    t, n, d = 128, 64 * 128, 64
+    m = xt.convert(_own_keys, args=(xt.Array((n, d), xt.float16), xt.Array((n, d), xt.float16), xt.Array((n, d), xt.float32),
+                                    xt.Array((n, d), xt.float32), t, d, t), grid=(n // t, 1, 1))
+    bufs = _inputs(11, (n, d), (n, d), (n, d), "f16")
+    want = run_oracle(m, bufs, oracle_threads())[3]
+    dev = [to_device(x, dt, cuda) for x, dt in zip(bufs, ("f16", "f16", "f32", "f32"))]
+    print(f"[gpu] attention over its values, {how}", flush=True)
+    if how == "one memref":
+        over_v = str(m).replace("%matmul2, %output,", "%matmul2, %input3,")
+        assert over_v != str(m) and " attention waves=" not in xt.plan(xt.parse(over_v))["kernel"]
+        xt.launch(xt.parse(over_v), *dev)
+    else:
+        xt.launch(m, dev[0], dev[1], dev[2], dev[2])
+    torch.cuda.synchronize()
+    assert frob_rel(dev[2].cpu().numpy(), want) <= 1e-5

@@ -400,3 +400,29 @@ def test_in_place_programs_must_touch_only_their_own_tile():
     transposed = INDEPENDENCE.format(load="%bid#0, %bid#1", store="%bid#1, %bid#0").replace("%c,", "%a,")
     with pytest.raises(NotImplementedError, match="stored and also accessed at another tile"):
         xt.plan(xt.parse(transposed))
+
+
+@xt.kernel
+def _attend_own_keys(q, k, v, o, tq, nk, d):
+    i = xt.bid(0)
+    qt = xt.load(q, index=(i, 0), shape=(tq, d))
+    kt = xt.load(k, index=(i, 0), shape=(nk, d))
+    vt = xt.load(v, index=(i, 0), shape=(nk, d))
+    s = xt.matmul(qt, xt.reshape(xt.transpose(xt.reshape(kt, shape=(1, nk, d))), shape=(d, nk)))
+    p = xt.exp(xt.sub(s, xt.max(s, axis=1)))
+    p = xt.mul(p, xt.reciprocal(xt.sum(p, axis=1)))
+    xt.store(o, index=(i, 0), tile=xt.matmul(p, vt))
+
+
+def test_attention_over_its_own_values_stays_staged():
+    """softmax(Q K^T) V stored back into V: the attention kernel's workgroups
+    share a Block's V, so the program keeps the staged kernel's one workgroup a
+    Block."""
+    n, t, d = 512, 128, 64
+    h, f = xt.Array((n, d), xt.float16), xt.Array((n, d), xt.float32)
+    apart = xt.convert(_attend_own_keys, args=(h, h, f, f, t, t, d), grid=(n // t, 1, 1))
+    assert " attention waves=" in xt.plan(apart)["kernel"]
+    over_v = str(apart).replace("%matmul2, %output,", "%matmul2, %input3,")
+    assert over_v != str(apart)
+    kernel = xt.plan(xt.parse(over_v))["kernel"]
+    assert kernel.startswith("staged") and " attention waves=" not in kernel

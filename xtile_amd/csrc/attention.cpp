@@ -304,6 +304,10 @@ extern "C" __global__ void __launch_bounds__(64 * NW) xt_attend(FusedArgs a) {
 bool attend_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& fp) {
   Form f;
   if (!match(vm, f)) return false;
+  // Several workgroups read a head's K and V while others store its rows: O is a
+  // memref of its own (buffers that meet: launch_fused).  A Block that updates
+  // its own tile in place stays with the staged kernel, one workgroup a Block.
+  if (f.o->arg == f.v->arg || f.o->arg == f.k->arg || f.o->arg == f.q->arg) return false;
   if ((f.q->elem != Elem::F16 && f.q->elem != Elem::BF16) || f.k->elem != f.q->elem || f.v->elem != Elem::F32 ||
       f.o->elem != Elem::F32)
     return false;

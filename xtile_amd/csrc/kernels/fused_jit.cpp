@@ -177,7 +177,12 @@ hipError_t launch_fused(const xt::Plan& p, void* const* bufs, hipStream_t s, std
   // that variant does not fit the fused layout.
   uintptr_t align = 0;
   bool attend = fp->attend_workgroups > 0;
-  for (const xt::VmAccess& a : vm.access) attend = attend && reinterpret_cast<uintptr_t>(bufs[a.arg]) % 16 == 0;
+  if (attend) {  // xt_attend's stores must not meet what other workgroups still read
+    const int out = vm.access[vm.inst.back().kind].arg;  // the program ends with its store
+    for (const xt::VmAccess& a : vm.access)
+      attend = attend && reinterpret_cast<uintptr_t>(bufs[a.arg]) % 16 == 0 &&
+               (a.arg == out || !buffers_meet(p, bufs, a.arg, out));
+  }
   int bad = attend ? -1 : misaligned(vm, bufs, fp->vw, align);
   if (bad >= 0 && fp->vw > 1) {
     std::string err;

@@ -53,6 +53,16 @@ inline bool ksplit_allowed() {
   return !(v && v[0] == '0' && v[1] == '\0');
 }
 
+// Whether the buffers of two memref arguments share a byte (one tensor may be
+// passed for both).
+inline bool buffers_meet(const xt::Plan& p, void* const* bufs, int i, int j) {
+  auto at = [&](int k) { return reinterpret_cast<uintptr_t>(bufs[k]); };
+  auto end = [&](int k) {
+    return at(k) + static_cast<uintptr_t>(p.arg_types[k].numel()) * xt::elem_bytes(p.arg_types[k].elem);
+  };
+  return at(i) < end(j) && at(j) < end(i);
+}
+
 // Blocks of the plan's grid, in 64 bits (three int32 axes).
 inline long long grid_blocks(const xt::Plan& p) {
   return static_cast<long long>(p.grid[0]) * p.grid[1] * p.grid[2];

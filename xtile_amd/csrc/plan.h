@@ -109,7 +109,8 @@ struct FusedPlan {
   std::shared_ptr<FusedPlan> scalar;
   bool staged = false;       // written by stage_vm (values in LDS), not fuse_vm
   // a staged program whose source also holds attend_vm's kernel `xt_attend`,
-  // which runs when every buffer is 16-byte aligned (0 workgroups: none)
+  // which runs when every buffer is 16-byte aligned and the result's meets no
+  // other (0 workgroups: none)
   int attend_threads = 0, attend_workgroups = 0;
 };
 

@@ -51,7 +51,7 @@
 // The first consumer in program order decides.
 //
 // Attention programs carry a second kernel beside this one (attention.cpp), which
-// runs when the buffers are 16-byte aligned.
+// runs when the buffers are 16-byte aligned and the result's meets no other.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
