@@ -17,6 +17,7 @@ import xtile_amd as xt
 from oracle import bf16_bits_to_f32, closed_form, f32_to_bf16_bits
 from tests.conftest import oracle_threads
 from tests.gpu_util import frob_rel, run_gpu, run_oracle, to_device
+from tests.test_plan import i8_over
 from xtile_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
@@ -126,3 +127,50 @@ def test_buffers_off_the_vector_alignment(cuda):
     xt.launch(mod, *dev)
     torch.cuda.synchronize()
     assert frob_rel(dev[2].cpu().numpy(), closed_form.matmul(_wide(a), _wide(b))) <= _bar(k)
+
+
+@pytest.mark.parametrize("how", ["one memref", "one tensor"])
+@pytest.mark.parametrize("operand,blocks,t,n", [("a", 25, 40, 100), ("a", 64, 24, 132), ("b", 9, 40, 100)])
+def test_i8_products_over_an_operand(cuda, how, operand, blocks, t, n):
+    """Each Block's product stored over its own tile of A or B, as one memref of
+    the program and as one tensor passed for both: the oracle's bytes of the
+    product stored elsewhere."""
+    import torch
+
+    apart, over = i8_over(operand, blocks, t, n)
+    rng = np.random.default_rng(n)
+    shape = {"a": [(blocks * t, n), (n, n)], "b": [(n, n), (n, blocks * t)]}[operand]
+    a, b = (rng.integers(-3, 4, s, dtype=np.int8) for s in shape)
+    at = "ab".index(operand)
+    want = run_oracle(apart, [a, b, np.zeros_like((a, b)[at])], oracle_threads())[2]
+    dev = [to_device(x, "i8", cuda) for x in (a, b, np.zeros_like((a, b)[at]))]
+    print(f"[gpu] i8 product over {operand}, {how}: {xt.plan(over)['kernel']}", flush=True)
+    if how == "one memref":
+        xt.launch(over, *dev)
+    else:
+        xt.launch(apart, dev[0], dev[1], dev[at])
+    torch.cuda.synchronize()
+    assert np.array_equal(dev[at].cpu().numpy(), want)
+
+
+def test_one_row_over_its_bias(cuda):
+    """c = a @ b + c over one row, c of two column Blocks: the sum's own memref as
+    the bias."""
+    k, n, tn = 72, 180, 90
+    m = xt.convert(_row_plus_kernel, args=(xt.Array((1, k), xt.float16), xt.Array((k, n), xt.float16),
+                                          xt.Array((1, n), xt.float32), k, tn), grid=(2, 1, 1))
+    assert " gemm k=72" in xt.plan(m)["kernel"]
+    rng = np.random.default_rng(2)
+    a, b = _narrow(rng, (1, k), "f16"), _narrow(rng, (k, n), "f16")
+    c = rng.uniform(-1, 1, (1, n)).astype(np.float32)
+    got = run_gpu(m, [a, b, c], ["f16", "f16", "f32"], cuda, case="one row over its bias")[2]
+    assert frob_rel(got, closed_form.matmul(_wide(a), _wide(b)) + c) <= _bar(k)
+
+
+@xt.kernel
+def _row_plus_kernel(a, b, c, k, tn):
+    j = xt.bid(0)
+    x = xt.load(a, index=(0, 0), shape=(1, k), shared=1)
+    w = xt.load(b, index=(0, j), shape=(k, tn))
+    bias = xt.load(c, index=(0, j), shape=(1, tn))
+    xt.store(c, index=(0, j), tile=xt.matmul(x, w) + bias)

@@ -426,3 +426,43 @@ def test_attention_over_its_own_values_stays_staged():
     assert over_v != str(apart)
     kernel = xt.plan(xt.parse(over_v))["kernel"]
     assert kernel.startswith("staged") and " attention waves=" not in kernel
+
+
+@xt.kernel
+def i8_row_blocks(a, b, o, tm, k, n):
+    i = xt.bid(0)
+    x = xt.load(a, index=(i, 0), shape=(tm, k))
+    w = xt.load(b, index=(0, 0), shape=(k, n), shared=1)
+    xt.store(o, index=(i, 0), tile=xt.astype(xt.matmul(x, w), dtype=xt.int8))
+
+
+@xt.kernel
+def i8_column_blocks(a, b, o, m, k, tn):
+    i = xt.bid(0)
+    x = xt.load(a, index=(0, 0), shape=(m, k), shared=1)
+    w = xt.load(b, index=(0, i), shape=(k, tn))
+    xt.store(o, index=(0, i), tile=xt.astype(xt.matmul(x, w), dtype=xt.int8))
+
+
+def i8_over(operand, blocks, t, n):
+    """(module, module that stores over its own operand): `blocks` products of t
+    rows of A with the n x n B, or of the n x n A with t columns of B."""
+    i8 = lambda *shape: xt.Array(shape, xt.int8)  # noqa: E731
+    if operand == "a":
+        m = xt.convert(i8_row_blocks, args=(i8(blocks * t, n), i8(n, n), i8(blocks * t, n), t, n, n), grid=(blocks, 1, 1))
+    else:
+        m = xt.convert(i8_column_blocks, args=(i8(n, n), i8(n, blocks * t), i8(n, blocks * t), n, n, t), grid=(blocks, 1, 1))
+    text = str(m).replace("%cast, %output,", "%cast, %input," if operand == "a" else "%cast, %input2,")
+    assert text != str(m)
+    return m, xt.parse(text)
+
+
+@pytest.mark.parametrize("operand,blocks,t,n", [("a", 25, 40, 100), ("b", 3, 40, 100)])
+def test_ragged_products_over_an_operand_stay_staged(operand, blocks, t, n):
+    """A Block's product stored over its own tile of A or B: the GEMM kernel's
+    tiles would read rows or columns that others store, so it keeps the staged
+    kernel's one workgroup a Block."""
+    apart, over = i8_over(operand, blocks, t, n)
+    assert f" gemm k={n}" in xt.plan(apart)["kernel"]
+    kernel = xt.plan(over)["kernel"]
+    assert kernel.startswith("staged") and " gemm k=" not in kernel

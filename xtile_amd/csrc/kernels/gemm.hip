@@ -811,6 +811,13 @@ bool launch_gemm_ragged(const xt::Plan& p, void* const* bufs, hipStream_t s, hip
   const long long es = i8 ? 1 : 2;
   int64_t M, N;
   if (!xt::gemm_region(p, M, N) || M >= (1LL << 31) || N >= (1LL << 31) || p.gemm_k >= (1LL << 17)) return false;
+  // a result over its operands stays staged, one workgroup a Block; over the
+  // epilogue's rows it may lie where it is one row, which the thread that
+  // stores a column read at that column before
+  if (accesses_meet(p, bufs, p.c, p.a) || accesses_meet(p, bufs, p.c, p.b) ||
+      (M > 1 && ((p.gemm_scale && accesses_meet(p, bufs, p.c, p.scale)) ||
+                 (p.gemm_bias && accesses_meet(p, bufs, p.c, p.bias)))))
+    return false;
   auto origin = [&](const xt::Access2D& v, long long b) { return static_cast<unsigned char*>(bufs[v.arg]) + v.addr.c0 * b; };
   auto aligned = [](const void* q, long long n) { return reinterpret_cast<uintptr_t>(q) % n == 0; };
   const unsigned char *A = origin(p.a, es), *B = origin(p.b, es), *C = origin(p.c, out_i8 ? 1 : 4);

@@ -63,6 +63,20 @@ inline bool buffers_meet(const xt::Plan& p, void* const* bufs, int i, int j) {
   return at(i) < end(j) && at(j) < end(i);
 }
 
+// Whether the bytes that all Blocks touch of two accesses, as ranges, meet: one
+// memref, or one tensor passed for two.
+inline bool accesses_meet(const xt::Plan& p, void* const* bufs, const xt::Access2D& x, const xt::Access2D& y) {
+  auto first = [&](const xt::Access2D& v) {
+    return reinterpret_cast<uintptr_t>(bufs[v.arg]) + static_cast<uintptr_t>(v.addr.c0) * xt::elem_bytes(v.elem);
+  };
+  auto past = [&](const xt::Access2D& v) {  // tile steps and pitches are not negative
+    const long long n = (p.grid[0] - 1) * v.addr.sx + (p.grid[1] - 1) * v.addr.sy + (p.grid[2] - 1) * v.addr.sz +
+                        (v.rows - 1) * v.ld + v.cols;
+    return first(v) + static_cast<uintptr_t>(n) * xt::elem_bytes(v.elem);
+  };
+  return first(x) < past(y) && first(y) < past(x);
+}
+
 // Blocks of the plan's grid, in 64 bits (three int32 axes).
 inline long long grid_blocks(const xt::Plan& p) {
   return static_cast<long long>(p.grid[0]) * p.grid[1] * p.grid[2];

@@ -1045,11 +1045,14 @@ bool build_plan(const Module& m, const std::string& func, Plan& p, std::string& 
     std::string why, why_staged;
     if (!fuse_off && (fuse_vm(p.vm, p.grid, fp, why) ||
                       (!(stage_env && std::string(stage_env) == "0") && stage_vm(p.vm, p.grid, fp, why_staged)))) {
-      // a staged product whose sizes the GEMM form above refuses
+      // a staged product whose sizes the GEMM form above refuses, stored
+      // elsewhere than over A or B: the GEMM kernel's tiles share their rows
+      // and columns, a staged Block has its own in LDS before it stores
       Plan q = p;
       std::string e2;
       int64_t M, N;
-      if (fp.staged && match_gemm_form(an, q, e2, true) && gemm_region(q, M, N) && q.gemm_k < (int64_t(1) << 17)) {
+      if (fp.staged && match_gemm_form(an, q, e2, true) && gemm_region(q, M, N) && q.gemm_k < (int64_t(1) << 17) &&
+          q.c.arg != q.a.arg && q.c.arg != q.b.arg) {
         p.a = q.a;
         p.b = q.b;
         p.c = q.c;
