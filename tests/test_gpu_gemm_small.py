@@ -130,7 +130,9 @@ def test_buffers_off_the_vector_alignment(cuda):
 
 
 @pytest.mark.parametrize("how", ["one memref", "one tensor"])
-@pytest.mark.parametrize("operand,blocks,t,n", [("a", 25, 40, 100), ("a", 64, 24, 132), ("b", 9, 40, 100)])
+@pytest.mark.parametrize("operand,blocks,t,n", [("a", 25, 40, 100), ("a", 64, 24, 132), ("b", 9, 40, 100),
+                                                 ("a", 8, 128, 128), ("a", 6, 64, 256), ("a", 5, 192, 128), ("b", 7, 128, 128),
+                                                 ("b", 5, 64, 256)])
 def test_i8_products_over_an_operand(cuda, how, operand, blocks, t, n):
     """Each Block's product stored over its own tile of A or B, as one memref of
     the program and as one tensor passed for both: the oracle's bytes of the

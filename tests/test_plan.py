@@ -466,3 +466,28 @@ def test_ragged_products_over_an_operand_stay_staged(operand, blocks, t, n):
     assert f" gemm k={n}" in xt.plan(apart)["kernel"]
     kernel = xt.plan(over)["kernel"]
     assert kernel.startswith("staged") and " gemm k=" not in kernel
+
+
+@pytest.mark.parametrize("operand,blocks,t,n", [("a", 8, 128, 128), ("a", 3, 512, 256), ("a", 3, 64, 128), ("a", 2, 192, 128),
+                                                ("b", 4, 128, 256), ("b", 3, 64, 128)])
+def test_products_over_an_operand(operand, blocks, t, n):
+    """Stored over its own tile of A or B, a product runs on the GEMM kernel where
+    a tile of it, with edges or without, takes whole Blocks along that operand."""
+    assert xt.plan(i8_over(operand, blocks, t, n)[1])["kernel"].startswith("gemm")
+
+
+def test_products_over_an_operand_with_a_b_of_each_block_are_staged():
+    """64-row Blocks with a B each: only 64-row tiles take them, which split the
+    128 columns."""
+    m = xt.convert(i8_row_blocks, args=(xt.Array((192, 128), xt.int8), xt.Array((384, 128), xt.int8),
+                                       xt.Array((192, 128), xt.int8), 64, 128, 128), grid=(3, 1, 1))
+    text = str(m).replace("%input2, %zero, %zero", "%input2, %bid#0, %zero").replace("{shared = 1 : i64} ", "")
+    assert xt.plan(xt.parse(text))["kernel"].startswith("gemm")
+    assert xt.plan(xt.parse(text.replace("%cast, %output,", "%cast, %input,")))["kernel"].startswith("staged")
+
+
+def test_products_over_an_operand_wider_than_any_tile_are_refused():
+    apart, over = i8_over("a", 4, 64, 512)
+    assert xt.plan(apart)["kernel"].startswith("gemm")
+    with pytest.raises(NotImplementedError, match="stores over its own operand"):
+        xt.plan(over)

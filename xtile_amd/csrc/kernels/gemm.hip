@@ -461,54 +461,6 @@ bool offs_multiple(const xt::TileAddr& a, long long m) {
   return a.c0 % m == 0 && a.sx % m == 0 && a.sy % m == 0 && a.sz % m == 0;
 }
 
-long long axis_step(const xt::TileAddr& a, int axis) {
-  return axis == 0 ? a.sx : axis == 1 ? a.sy : a.sz;
-}
-
-// How one workgroup tile of `w` elements covers Blocks of `t` elements along
-// M (is_m) or N: split (sub > 1), exact, or fused over `factor` neighbouring
-// Blocks along a grid axis whose next Block continues the same rows/columns.
-struct Cover {
-  bool ok = false;
-  int sub = 1;
-  int axis = -1;
-  int factor = 1;
-};
-
-Cover cover_dim(const xt::Plan& p, long long w, bool is_m) {
-  Cover c;
-  const long long t = is_m ? p.a.rows : p.b.cols;
-  if (t % w == 0) {
-    c.ok = true;
-    c.sub = static_cast<int>(t / w);
-    return c;
-  }
-  if (w % t) return c;
-  const int f = static_cast<int>(w / t);
-  for (int ax = 0; ax < 3; ++ax) {
-    if (p.grid[ax] % f) continue;
-    // the epilogue rows follow B's columns
-    const bool rows_fixed = (!p.gemm_scale || axis_step(p.scale.addr, ax) == 0) &&
-                            (!p.gemm_bias || axis_step(p.bias.addr, ax) == 0);
-    const bool rows_follow = (!p.gemm_scale || axis_step(p.scale.addr, ax) == t) &&
-                             (!p.gemm_bias || axis_step(p.bias.addr, ax) == t);
-    bool contiguous;
-    if (is_m)
-      contiguous = axis_step(p.c.addr, ax) == t * p.c.ld && axis_step(p.a.addr, ax) == t * p.a.ld &&
-                   axis_step(p.b.addr, ax) == 0 && rows_fixed;
-    else
-      contiguous = axis_step(p.c.addr, ax) == t && axis_step(p.b.addr, ax) == t &&
-                   axis_step(p.a.addr, ax) == 0 && rows_follow;
-    if (contiguous) {
-      c.ok = true;
-      c.axis = ax;
-      c.factor = f;
-      return c;
-    }
-  }
-  return c;
-}
-
 // Zero-fills rows x (4 cols4) floats at pitch ld (a kernel, not
 // hipMemsetAsync, so that a captured graph replays it correctly).
 __global__ __launch_bounds__(256) void gemm_zero_kernel(float* __restrict__ c, long long ld, int rows, int cols4) {
@@ -660,6 +612,8 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
   const bool region = xt::gemm_region(p, M, N) && M < (1LL << 31) && N < (1LL << 31);
   const bool can_split = ksplit_allowed() && !i8 && !out_i8 && !p.gemm_scale && !p.gemm_bias && region && N % 4 == 0 &&
                          p.c.ld % 4 == 0 && reinterpret_cast<uintptr_t>(cbase) % 16 == 0 && M < (1LL << 31);
+  // a result over A's or B's bytes: see gemm_tile
+  const bool over_a = accesses_meet(p, bufs, p.c, p.a), over_b = accesses_meet(p, bufs, p.c, p.b);
   // Workgroup tile, all on the DMA kernel: 256 x 256 when the Blocks map onto
   // it and its tiles fill the CUs, or are few enough for the K split below;
   // else the first of 256 x 128, 128 x 256, 128 x 128 whose tiles fill the
@@ -667,16 +621,16 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
   // 256 x 256, 256 of 128 x 128).
   struct Cand {
     int bm = 0, bn = 0;
-    Cover cm, cn;
+    xt::GemmCover cm, cn;
     long long tiles = 0;
     bool edge = false;  // tiles of the whole region, the last ones reaching past it
   };
   auto try_tile = [&](int bmv, int bnv, Cand& c) {
     c.bm = bmv;
     c.bn = bnv;
-    c.cm = cover_dim(p, bmv, true);
-    c.cn = cover_dim(p, bnv, false);
-    if (!c.cm.ok || !c.cn.ok || (c.cm.axis >= 0 && c.cm.axis == c.cn.axis)) return false;
+    c.cm = xt::gemm_cover(p, bmv, true);
+    c.cn = xt::gemm_cover(p, bnv, false);
+    if (!xt::gemm_tile(c.cm, c.cn, over_a, over_b)) return false;
     long long g[3] = {p.grid[0], p.grid[1], p.grid[2]};
     if (c.cm.axis >= 0) g[c.cm.axis] /= c.cm.factor;
     if (c.cn.axis >= 0) g[c.cn.axis] /= c.cn.factor;
@@ -732,7 +686,7 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
     }
     for (int t : {128, 256}) {
       Cand c;
-      if (!region || try_tile(t, t, c) || t * a.lda * es >= (1LL << 32)) continue;
+      if (!region || (over_a && N > t) || (over_b && M > t) || try_tile(t, t, c) || t * a.lda * es >= (1LL << 32)) continue;
       c = Cand{};
       c.bm = c.bn = t;
       c.edge = true;
@@ -740,12 +694,13 @@ hipError_t launch_gemm(const xt::Plan& p, void* const* bufs, hipStream_t s, std:
       offer(c);
     }
     if (pick.bm == 0) {
-      why = "matmul Blocks cannot be mapped onto workgroup tiles in one launch";
+      why = over_a || over_b ? "a matmul over the bytes of its own operand needs Blocks that workgroup tiles cover whole"
+                             : "matmul Blocks cannot be mapped onto workgroup tiles in one launch";
       return hipErrorInvalidValue;
     }
   }
   const int bm = pick.bm, bn = pick.bn;
-  const Cover cm = pick.cm, cn = pick.cn;
+  const xt::GemmCover cm = pick.cm, cn = pick.cn;
   a.mul[0] = a.mul[1] = a.mul[2] = 1;
   int vg[3] = {p.grid[0], p.grid[1], p.grid[2]};
   if (cm.axis >= 0) {

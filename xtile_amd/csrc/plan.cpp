@@ -491,6 +491,18 @@ bool match_gemm_form(const Analysis& an, Plan& p, std::string& err, bool ragged)
     err = "the HIP matmul kernel needs 16-byte aligned rows";
     return false;
   }
+  const bool over_a = p.c.arg == p.a.arg, over_b = p.c.arg == p.b.arg;
+  if (!ragged && (over_a || over_b)) {
+    int64_t RM, RN;  // a tile of the whole region may reach past its edges
+    bool fits = gemm_region(p, RM, RN) && (!over_a || RN <= 256) && (!over_b || RM <= 256);
+    for (int bm : {128, 256})  // the widest tiles of the kernel
+      for (int bn : {128, 256}) fits = fits || gemm_tile(gemm_cover(p, bm, true), gemm_cover(p, bn, false), over_a, over_b);
+    if (!fits) {
+      err = "the HIP matmul kernel stores over its own operand only where a workgroup tile, 256 wide at most, takes "
+            "whole Blocks along it";
+      return false;
+    }
+  }
   p.kind = PlanKind::Gemm;
   p.gemm_k = K;
   double blocks = double(p.grid[0]) * p.grid[1] * p.grid[2];
@@ -959,6 +971,45 @@ std::string Plan::describe() const {
   }
   os << " grid=(" << grid[0] << "," << grid[1] << "," << grid[2] << ")";
   return os.str();
+}
+
+GemmCover gemm_cover(const Plan& p, int64_t w, bool is_m) {
+  auto axis_step = [](const TileAddr& a, int axis) { return axis == 0 ? a.sx : axis == 1 ? a.sy : a.sz; };
+  GemmCover c;
+  const int64_t t = is_m ? p.a.rows : p.b.cols;
+  if (t % w == 0) {
+    c.ok = true;
+    c.sub = static_cast<int>(t / w);
+    return c;
+  }
+  if (w % t) return c;
+  const int f = static_cast<int>(w / t);
+  for (int ax = 0; ax < 3; ++ax) {
+    if (p.grid[ax] % f) continue;
+    // the epilogue rows follow B's columns
+    const bool rows_fixed = (!p.gemm_scale || axis_step(p.scale.addr, ax) == 0) &&
+                            (!p.gemm_bias || axis_step(p.bias.addr, ax) == 0);
+    const bool rows_follow = (!p.gemm_scale || axis_step(p.scale.addr, ax) == t) &&
+                             (!p.gemm_bias || axis_step(p.bias.addr, ax) == t);
+    bool contiguous;
+    if (is_m)
+      contiguous = axis_step(p.c.addr, ax) == t * p.c.ld && axis_step(p.a.addr, ax) == t * p.a.ld &&
+                   axis_step(p.b.addr, ax) == 0 && rows_fixed;
+    else
+      contiguous = axis_step(p.c.addr, ax) == t && axis_step(p.b.addr, ax) == t &&
+                   axis_step(p.a.addr, ax) == 0 && rows_follow;
+    if (contiguous) {
+      c.ok = true;
+      c.axis = ax;
+      c.factor = f;
+      return c;
+    }
+  }
+  return c;
+}
+
+bool gemm_tile(const GemmCover& m, const GemmCover& n, bool over_a, bool over_b) {
+  return m.ok && n.ok && (m.axis < 0 || m.axis != n.axis) && !(over_a && n.sub > 1) && !(over_b && m.sub > 1);
 }
 
 bool gemm_region(const Plan& p, int64_t& M, int64_t& N) {

@@ -174,6 +174,25 @@ bool attend_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& fp);
 // tile's columns (A fixed).
 bool gemm_region(const Plan& p, int64_t& M, int64_t& N);
 
+// How one workgroup tile of `w` elements covers a Gemm plan's Blocks of `t`
+// elements along M (is_m) or N: split (sub > 1), exact, or fused over `factor`
+// neighbouring Blocks along a grid axis whose next Block continues the same
+// rows / columns.
+struct GemmCover {
+  bool ok = false;
+  int sub = 1;
+  int axis = -1;
+  int factor = 1;
+};
+GemmCover gemm_cover(const Plan& p, int64_t w, bool is_m);
+
+// Whether tiles of these covers may run a Gemm plan.  Over its own operand's
+// bytes (over_a, over_b: C's tile is A's or B's, a Block's own) a workgroup has to
+// take whole Blocks along N (A) or M (B): it has all its rows of A (columns of
+// B) in LDS before it stores, and another tile of the Block would still read
+// them.
+bool gemm_tile(const GemmCover& m, const GemmCover& n, bool over_a, bool over_b);
+
 // Builds the plan of function `func` (empty name: the only function).
 // Returns false and sets `error` when the program is not one the HIP
 // backend runs.
