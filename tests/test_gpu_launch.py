@@ -76,6 +76,24 @@ def test_refusals(cuda):
     assert not c.any()
 
 
+def test_a_handle_is_known_by_its_type(cuda):
+    """An object with an address for a module, and a capsule of the compiled
+    binding while the ctypes one is in use, are refused by their type."""
+    from xtile_amd import _compiled
+
+    class Alike:
+        _ptr = 16
+
+    class Holder:
+        _CAPIPtr = Alike()
+
+    a, b, c = _buffers(cuda)
+    for handle in (Alike(), Holder(), _compiled.load().parse(xt._wrap_module_asm(str(K.add(64, 128)))[0])):
+        with pytest.raises(TypeError, match="expected an xtile module object"):
+            xt.launch(handle, a, b, c)
+    assert not c.any()
+
+
 def test_a_pass_drops_the_plan(cuda):
     """The plan a launch used is not kept across a pass over its module."""
     import torch

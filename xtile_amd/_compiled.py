@@ -59,6 +59,8 @@ def load_launch(native):
     spec.loader.exec_module(module)
     lib = getattr(native, "lib", None) or ctypes.CDLL(str(MODULE_PATH.with_name("libxtile_amd.so")))
     module.bind(
-        ctypes.cast(lib.xt_gpu_run_buffers, ctypes.c_void_p).value, ctypes.cast(lib.xt_free, ctypes.c_void_p).value
+        ctypes.cast(lib.xt_gpu_run_buffers, ctypes.c_void_p).value,
+        ctypes.cast(lib.xt_free, ctypes.c_void_p).value,
+        getattr(native, "NativeModule", None),  # the compiled binding's handles are capsules
     )
     return module.launch

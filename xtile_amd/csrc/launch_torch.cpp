@@ -5,8 +5,9 @@
 // us of host time, several times what a small kernel runs; this call takes the
 // tensors' fields from their C++ objects and hands them to xt_gpu_run_buffers.
 //
-//   bind(address)                        of xt_gpu_run_buffers in the library
-//                                        that owns the module handles
+//   bind(run, free, type)                xt_gpu_run_buffers and xt_free of the library
+//                                        that owns the module handles, as addresses,
+//                                        and the handles' type (None: capsules)
 //   launch(handle, buffers, func, stream) True when the program was enqueued.
 //                                        False when anything is not the plain
 //                                        case: the caller then takes the checked
@@ -35,17 +36,20 @@ typedef int (*RunFn)(xt_module*, const char*, const xt_buffer*, int, void*, char
 typedef void (*FreeFn)(void*);
 RunFn g_run = nullptr;
 FreeFn g_free = nullptr;
-PyObject* g_ptr_name = nullptr;  // "_ptr"
+PyTypeObject* g_handle = nullptr;  // the ctypes binding's NativeModule; nullptr: capsules
+PyObject* g_ptr_name = nullptr;    // "_ptr"
 
 constexpr const char* kCapsuleName = "xtile_amd.xt_module";
 constexpr int kMost = 16;
 
-// The module behind a ctypes handle (its `_ptr`) or a capsule; nullptr otherwise.
+// The module behind a handle of the binding in use; nullptr for anything else,
+// whatever attributes it has.
 xt_module* module_of(PyObject* handle) {
-  if (PyCapsule_CheckExact(handle))
+  if (!g_handle)
     return PyCapsule_IsValid(handle, kCapsuleName)
                ? static_cast<xt_module*>(PyCapsule_GetPointer(handle, kCapsuleName))
                : nullptr;
+  if (!PyObject_TypeCheck(handle, g_handle)) return nullptr;
   PyObject* p = PyObject_GetAttr(handle, g_ptr_name);
   if (!p) {
     PyErr_Clear();
@@ -161,13 +165,20 @@ PyObject* launch(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 }
 
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-  void* run = nargs == 2 && PyLong_Check(args[0]) ? PyLong_AsVoidPtr(args[0]) : nullptr;
-  void* release = nargs == 2 && PyLong_Check(args[1]) ? PyLong_AsVoidPtr(args[1]) : nullptr;
+  void* run = nargs == 3 && PyLong_Check(args[0]) ? PyLong_AsVoidPtr(args[0]) : nullptr;
+  void* release = nargs == 3 && PyLong_Check(args[1]) ? PyLong_AsVoidPtr(args[1]) : nullptr;
   if (PyErr_Occurred()) return nullptr;
-  if (!run || !release) {
-    PyErr_SetString(PyExc_ValueError, "bind(address of xt_gpu_run_buffers, address of xt_free)");
+  if (!run || !release || (args[2] != Py_None && !PyType_Check(args[2]))) {
+    PyErr_SetString(PyExc_ValueError, "bind(address of xt_gpu_run_buffers, address of xt_free, handle type or None)");
     return nullptr;
   }
+  PyObject* const was = reinterpret_cast<PyObject*>(g_handle);
+  g_handle = nullptr;
+  if (args[2] != Py_None) {
+    Py_INCREF(args[2]);
+    g_handle = reinterpret_cast<PyTypeObject*>(args[2]);
+  }
+  Py_XDECREF(was);
   g_run = reinterpret_cast<RunFn>(run);
   g_free = reinterpret_cast<FreeFn>(release);
   Py_RETURN_NONE;
@@ -177,7 +188,7 @@ PyMethodDef kMethods[] = {
     {"launch", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(launch)), METH_FASTCALL,
      "launch(handle, buffers, func, stream) -> bool: whether the program was enqueued"},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(bind)), METH_FASTCALL,
-     "bind(xt_gpu_run_buffers, xt_free): the library's functions, as addresses"},
+     "bind(xt_gpu_run_buffers, xt_free, type): the library's functions, as addresses, and its handles' type"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_launch", "xt.launch over torch tensors", -1, kMethods,
