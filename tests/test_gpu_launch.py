@@ -18,7 +18,7 @@ def _buffers(cuda):
     return a, b, torch.zeros(64, 128, device=cuda)
 
 
-@pytest.mark.parametrize("how", ["plain", "func", "int", "object", "current", "subclass"])
+@pytest.mark.parametrize("how", ["plain", "func", "int", "object", "current", "subclass", "not built"])
 def test_launches(cuda, monkeypatch, how):
     import torch
 
@@ -29,6 +29,8 @@ def test_launches(cuda, monkeypatch, how):
     run = xt._launch_checked
     monkeypatch.setattr(xt, "_launch_checked", lambda *x: (checked.append(how), run(*x)))
     print(f"[gpu] launch {how}", flush=True)
+    if how == "not built":  # what _load_launch returns then
+        monkeypatch.setattr(xt, "_launch_native", lambda *_: False)
     if how == "func":
         xt.launch(m, a, b, c, func="add_kernel")
     elif how == "int":
@@ -47,7 +49,7 @@ def test_launches(cuda, monkeypatch, how):
         xt.launch(m, a, b, c)
     torch.cuda.synchronize()
     assert torch.equal(c, a + b)
-    assert checked == (["subclass"] if how == "subclass" else [])
+    assert checked == ([how] if how in ("subclass", "not built") else [])
 
 
 def test_refusals(cuda):

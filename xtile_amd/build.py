@@ -168,13 +168,23 @@ def launch_path() -> Path:
     return LIB / ("_launch" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 
-def build_launch() -> Path:
+def build_launch() -> Path | None:
     """Compile csrc/launch_torch.cpp against the installed torch.  It is handed
-    the library's entry points at run time, so it links torch only."""
-    import torch
-    from torch.utils import cpp_extension
-
+    the library's entry points at run time, so it links torch only.  None, and
+    an earlier build's module is gone, where torch or its headers are not
+    installed: xt.launch then checks its arguments in Python."""
     out = launch_path()
+    try:
+        import torch
+        from torch.utils import cpp_extension
+
+        headers = any((Path(p) / "ATen" / "core" / "Tensor.h").exists() for p in cpp_extension.include_paths("cuda"))
+    except ImportError:
+        headers = False
+    if not headers:
+        print("torch's C++ headers are not installed: xt.launch is built without its native call")
+        out.unlink(missing_ok=True)
+        return None
     tmp = out.with_name(out.name + ".tmp")
     _run(
         [
