@@ -428,6 +428,21 @@ def test_attention_over_its_own_values_stays_staged():
     assert kernel.startswith("staged") and " attention waves=" not in kernel
 
 
+@pytest.mark.parametrize("name,dt", [("input", "f16"), ("input2", "f16"), ("input3", "f32"), ("output", "f32")])
+def test_attention_over_rows_of_more_than_an_int_stays_staged(name, dt):
+    """Rows 3 * 2^30 elements apart in any of its arrays: the attention kernel's
+    pitches are ints."""
+    t, d = 16, 64
+    h, f = xt.Array((t, d), xt.float16), xt.Array((t, d), xt.float32)
+    text = str(xt.convert(_attend_own_keys, args=(h, h, f, f, t, t, d), grid=(1, 1, 1)))
+    assert " attention waves=" in xt.plan(xt.parse(text))["kernel"]
+    old, new = f"memref<{t}x{d}x{dt}>", f"memref<{t}x{3 << 30}x{dt}>"
+    lines = text.replace(f"%{name}: {old}", f"%{name}: {new}").splitlines()
+    wide = "\n".join(x.replace(old, new) if f"%{name}, %bid" in x else x for x in lines)
+    kernel = xt.plan(xt.parse(wide))["kernel"]
+    assert kernel.startswith("staged") and " attention waves=" not in kernel
+
+
 @xt.kernel
 def i8_row_blocks(a, b, o, tm, k, n):
     i = xt.bid(0)

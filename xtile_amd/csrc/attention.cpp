@@ -316,6 +316,8 @@ bool attend_vm(const VmPlan& vm, const int32_t grid[3], FusedPlan& fp) {
   const long long ldk = f.k->stride[1], ldv = f.v->stride[1];
   const int kp = (f.nk + 15) / 16 * 16;
   const long long lds = (long long)kp * f.d * 6;
+  // the kernel holds every pitch in an int
+  if (f.q->stride[1] >= (1LL << 31) || f.o->stride[1] >= (1LL << 31)) return false;
   if (lds > kLds || f.nk > 512 || ldk * 2 * f.nk >= (1LL << 31) || ldv * 4 * f.nk >= (1LL << 31)) return false;
   // the grid axis whose Blocks continue the query rows of one head
   int rows_axis = -1;
