@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+import ctypes
+import re
 import sys
 
 import numpy as np
@@ -28,8 +30,9 @@ def to_host(t, dtype: str) -> np.ndarray:
     return t.numpy()
 
 
-def run_gpu(module, host_buffers, dtypes, device, func=None, case: str = ""):
-    """Copy buffers to the GPU, launch, synchronise, return host copies."""
+def run_gpu(module, host_buffers, dtypes, device, func=None, case: str = "", kernels=None):
+    """Copy buffers to the GPU, launch, synchronise, return host copies.  With
+    `kernels`, the launch has to enqueue exactly these (kernels_of)."""
     import torch
 
     import xtile_amd as xt
@@ -39,7 +42,36 @@ def run_gpu(module, host_buffers, dtypes, device, func=None, case: str = ""):
     dev = [to_device(b, d, device) for b, d in zip(host_buffers, dtypes)]
     xt.launch(module, *dev, func=func)
     torch.cuda.synchronize()
-    return [to_host(t, d) for t, d in zip(dev, dtypes)]
+    got = [to_host(t, d) for t, d in zip(dev, dtypes)]
+    if kernels is not None:
+        assert kernels_of(module, dev, func) == kernels
+    return got
+
+
+def kernels_of(module, buffers, func=None) -> list[str]:
+    """The kernels a launch of `module` over these device buffers enqueues, as
+    name<template arguments>, read from a graph that captures it."""
+    import tempfile
+
+    import torch
+
+    import xtile_amd as xt
+
+    xt.launch(module, *buffers, func=func)  # what a first launch loads stays out of the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        xt.launch(module, *buffers, func=func)
+    hip = ctypes.CDLL(next(x.split()[-1] for x in open("/proc/self/maps") if "libamdhip64" in x))
+    with tempfile.NamedTemporaryFile("r", suffix=".dot") as dot:
+        assert hip.hipGraphDebugDotPrint(ctypes.c_void_p(graph.raw_cuda_graph()), dot.name.encode(), 1) == 0
+        mangled = re.findall(r"(\w+)\\<\\<\\<", dot.read())
+    names = []
+    for name in mangled:  # a symbol of the library's, or a generated kernel's name
+        m = re.search(r"_GLOBAL__N_1\d+([a-z]\w*?)(?:I((?:L[a-z]\d+E)+))?E", name)
+        args = re.findall(r"L[a-z](\d+)E", m[2] or "") if m else []
+        names.append((m[1] if m else name) + (f"<{', '.join(args)}>" if args else ""))
+    return names
 
 
 def run_oracle(module, host_buffers, nthreads: int):

@@ -13,7 +13,7 @@ import pytest
 import xtile_amd as xt
 from oracle import f32_to_bf16_bits
 from tests.conftest import oracle_threads
-from tests.gpu_util import frob_rel, run_gpu, run_oracle, to_device
+from tests.gpu_util import frob_rel, kernels_of, run_gpu, run_oracle, to_device
 from xtile_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
@@ -30,7 +30,7 @@ def _inputs(seed, q, k, v, dt):
 
 def _check(cuda, m, bufs, dt, case):
     assert " attention waves=" in xt.plan(m)["kernel"]
-    got = run_gpu(m, bufs, [dt, dt, "f32", "f32"], cuda, case=case)[3]
+    got = run_gpu(m, bufs, [dt, dt, "f32", "f32"], cuda, case=case, kernels=["xt_attend"])[3]
     want = run_oracle(m, bufs, oracle_threads())[3]
     assert frob_rel(got, want) <= 1e-5
 
@@ -141,6 +141,7 @@ def test_buffers_off_the_alignment(cuda, off):
         flat[off : off + x.size] = t.reshape(-1)
         dev.append(flat[off : off + x.size].view(x.shape))
     print(f"[gpu] attention, buffers {off} elements off", flush=True)
+    assert kernels_of(m, dev) == ["xt_fused"]
     xt.launch(m, *dev)
     torch.cuda.synchronize()
     assert frob_rel(dev[3].cpu().numpy(), run_oracle(m, bufs, 1)[3]) <= 1e-5
@@ -160,6 +161,8 @@ def test_result_over_the_values(cuda, how):
     want = run_oracle(m, bufs, oracle_threads())[3]
     dev = [to_device(x, dt, cuda) for x, dt in zip(bufs, ("f16", "f16", "f32", "f32"))]
     print(f"[gpu] attention over its values, {how}", flush=True)
+    if how == "one tensor":
+        assert kernels_of(m, dev) == ["xt_attend"]
     if how == "one memref":
         over_v = str(m).replace("%matmul2, %output,", "%matmul2, %input3,")
         assert over_v != str(m) and " attention waves=" not in xt.plan(xt.parse(over_v))["kernel"]
@@ -168,3 +171,5 @@ def test_result_over_the_values(cuda, how):
         xt.launch(m, dev[0], dev[1], dev[2], dev[2])
     torch.cuda.synchronize()
     assert frob_rel(dev[2].cpu().numpy(), want) <= 1e-5
+    if how == "one tensor":
+        assert kernels_of(m, [dev[0], dev[1], dev[2], dev[2]]) == ["xt_fused"]

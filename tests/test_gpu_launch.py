@@ -106,3 +106,38 @@ def test_a_pass_drops_the_plan(cuda):
     with pytest.raises((NotImplementedError, ValueError)):
         xt.launch(m, a, b, c)
     torch.cuda.synchronize()
+
+
+def test_threads_on_one_module(cuda):
+    """Threads that plan and launch one module at once, each on a stream of its
+    own, through the native call (which holds no interpreter lock meanwhile)."""
+    import threading
+
+    import torch
+
+    for _ in range(4):
+        m = K.add(96, 640, 32, 64)  # planned by the first launch
+        sets = [(torch.rand(96, 640, device=cuda), torch.rand(96, 640, device=cuda), torch.zeros(96, 640, device=cuda))
+                for _ in range(8)]
+        streams = [torch.cuda.Stream() for _ in sets]
+        torch.cuda.synchronize()
+        start, failed = threading.Barrier(len(sets)), []
+
+        def work(bufs, stream):
+            try:
+                start.wait(timeout=30)
+                with torch.cuda.stream(stream):
+                    for _ in range(20):
+                        xt.launch(m, *bufs)
+                stream.synchronize()
+            except Exception as exc:  # noqa: BLE001
+                failed.append(exc)
+
+        threads = [threading.Thread(target=work, args=x) for x in zip(sets, streams)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=60)
+        assert not failed and not any(t.is_alive() for t in threads)
+        for a, b, c in sets:
+            assert torch.equal(c, a + b)

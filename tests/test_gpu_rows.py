@@ -10,6 +10,7 @@ import pytest
 
 import xtile_amd as xt
 from oracle import closed_form
+from tests.gpu_util import kernels_of
 from xtile_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +61,33 @@ def test_row_softmax(cuda, rows, cols, trow, off):
     x = rng.normal(0, 2, (rows, cols)).astype(np.float32)
     got = _run(cuda, K.softmax(rows, cols, trow), off, f"softmax {rows}x{cols}/{trow}", x, np.zeros_like(x))
     np.testing.assert_allclose(got, closed_form.softmax_rows(x), rtol=1e-5, atol=1.2e-38)
+
+
+@pytest.mark.parametrize("rows,cols,trow,kernel", [((1 << 32) + 4096, 2, 4096, "row_softmax_kernel<1, 1, 1>"),
+                                                  (8388611, 2048, 7, "row_softmax_wide_kernel<512, 1, 1>")])
+def test_row_softmax_of_more_rows_than_a_launch_takes(cuda, rows, cols, trow, kernel):
+    """More rows than 2^31 indices or one launch's 2^32 threads: the workgroups
+    walk them.  In place (34 and 69 GB); row r's odd columns stand r % 1021 / 256
+    above a row of its even ones, so a row written elsewhere shows."""
+    import torch
+
+    if torch.cuda.mem_get_info()[0] < rows * cols * 4 + (8 << 30):
+        pytest.skip("not enough free memory on the GPU")
+    base = torch.linspace(-1, 1, cols, device=cuda)
+    chunk = (1 << 28) // cols
+
+    def part(r0):
+        step = (torch.arange(r0, min(r0 + chunk, rows), device=cuda) % 1021).float() / 256
+        return base + step[:, None] * (torch.arange(cols, device=cuda) % 2)
+
+    x = torch.empty(rows, cols, device=cuda)
+    for r0 in range(0, rows, chunk):
+        x[r0 : r0 + chunk] = part(r0)
+    m = K.softmax(rows, cols, trow)
+    print(f"[gpu] softmax of {rows} rows", flush=True)
+    xt.launch(m, x, x)
+    for r0 in range(0, rows, chunk):
+        torch.testing.assert_close(x[r0 : r0 + chunk], torch.softmax(part(r0), dim=1), rtol=1e-5, atol=0)
+    assert kernels_of(m, [x, x]) == [kernel]
+    del x
+    torch.cuda.empty_cache()
