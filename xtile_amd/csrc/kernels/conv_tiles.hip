@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256, 1) void conv_tiles_kernel(CtArgs p) {
       for (int e = 0; e < 2; ++e) {
         const int k = 8 * s + T::a_chunk(lane, e);
         const int tap = p.d_cc(k), kh = p.d_kw(tap), kw = tap - kh * p.KW;
-        dih[e] = k < p.chunks ? kh * p.dh : 1 << 30;  // past K: outside every image
+        dih[e] = k < p.chunks ? kh * p.dh : 1 << 29;  // past K: outside every image, rows past M included
         diw[e] = kw * p.dw;
         const int c16 = (k - tap * p.cc) * 16;
         toff[e] = (unsigned)((kh * p.dh * p.W + diw[e]) * p.C * ES + (PART ? min(c16, p.C - 16) : c16));
