@@ -9,7 +9,9 @@
 // traffic.  The staged kernel of the same program (one Block a CU, scores and
 // probabilities through LDS, a barrier between phases) took 51.3 us a launch,
 // this one 15.6; 256 heads x 512 x 160 x 128 308 -> 58, 9 x 96 x 232 x 64 21.4 ->
-// 5.7, 1024 x 64 x 64 x 64 15.2 -> 12.7, and none of 30 sizes slower.  Raising
+// 5.7, 1024 x 64 x 64 x 64 15.2 -> 12.7, and none of 30 drawn sizes slower
+// (profiles/attention_staged_compare.txt).  The matrix pipes are busy 0.59 of the
+// first one's cycles (profiles/attention_256_xt_attend.txt).  Raising
 // half of the waves' priority, to set softmax against products, changed nothing.
 //
 //   * A workgroup holds one head's K (16 bits) and V (f32) in LDS, fetched once

@@ -560,7 +560,8 @@ bool conv_blocks_cover_output(const xt::Plan& p, long long es) {
 // and end and its operands at ~70 KB a us.  (Measured / estimated: 5 x 18^2 x 512
 // -> 32 3 x 3 / 2 i8 36.6 / 36.9 here, 7.1 / 7.7 in 32 x 32 tiles; 53 x 47^2 x 40
 // -> 64 5 x 5 / 2 30.6 / 26.5, 15.3 / 14.9 in 64 x 64; 32 x 28^2 x 128 -> 128 20.1
-// / 21.0, 30.8 / 26.9.)
+// / 21.0, 30.8 / 26.9.  40 other layers, of the kernel each chose, loader-wave
+// tiles among them: 0.86 to 1.34, median 0.98; profiles/tile_estimates.txt.)
 static double igemm_us(bool deep, int stages, long long nwg, long long ksplit, long long outputs, int cus) {
   const double load = std::max(1.0, 0.85 * double(nwg) / cus);
   return 5.2 + (deep ? 0.36 : 0.44) * stages / ksplit * load + (ksplit > 1 ? 2.5 + 2e-6 * outputs * ksplit : 0);

@@ -391,12 +391,18 @@ hipError_t launch_sc(bool big, int tasks_npr, long long wgs, size_t lds, hipStre
 
 }  // namespace
 
-// `ahead`: only the layers where this kernel is the faster of it and the implicit
-// GEMM: 20 bytes of channels, or up to 28 of a 1 x 1 filter, one channel tile,
-// enough output rows for eight workgroups a CU and rows that fill their chunks
-// (32 x 112^2 x 20 -> 64 3 x 3 39.0 us, 47.2 there; 32 x 112^2 x 24 -> 64 1 x 1
-// 20.0, 25.0; but 24 -> 32 3 x 3 44.6 against 39.0, 64 x 56^2 x 20 -> 64, rows of
-// 56 in chunks of 128, 37.0 against 25.0, and 8 x 112^2 x 20 -> 64 15.3, 13.8).
+// `ahead`: only the layers that this kernel keeps from the implicit GEMM, which is
+// the slower there or, in two of the shapes tried, the faster: 20 bytes of
+// channels, or up to 28 of a 1 x 1 filter, one channel tile, enough output rows
+// for eight workgroups a CU and rows that fill their chunks.  us here and there,
+// 32 images unless given: 112^2 x 20 -> 64 38.4, 45.2, -> 32 35.2, 37.3, -> 16
+// 34.8, 37.3; 5 x 5 -> 64 70.5, 80.9; 128^2 -> 64 40.8, 49.6; 16 x 224^2 -> 32
+// 64.6, 65.0; 20 x 112^2 -> 64 24.8, 25.4; 1 x 1 112^2 x 20 -> 64 20.6, 24.9, 24
+// -> 64 20.5, 25.1, 28 -> 64 23.6, 25.4, 16 x 224^2 x 24 -> 32 28.8, 31.5, 126^2 x
+// 28 -> 64 26.5, 27.0; the slower here are 224^2 x 20 -> 64 3 x 3 / 2 58.0, 44.0
+// and 1 x 1 112^2 x 28 -> 16 22.8, 18.3.  Outside the rule: 24 -> 32 3 x 3 44.6
+// against 39.0, 64 x 56^2 x 20 -> 64, rows of 56 in chunks of 128, 37.0 against
+// 25.0, and 8 x 112^2 x 20 -> 64 15.3, 13.8.
 bool launch_conv2d_small(const xt::Plan& p, void* const* bufs, hipStream_t s, bool ahead, hipError_t& e) {
   const xt::ConvPlan& c = p.conv;
   const bool i8 = c.elem == xt::Elem::I8;

@@ -520,7 +520,8 @@ static int cu_count() {
 // loop at the operand rate one CU reached, and its output at its share of HBM.
 // (64 x 64: 1024^3 f16 9.5 us measured, 9.2 estimated; 1024 x 1024 x 4096 21.0,
 // 20.1.  32 x 64: 256 x 2048 x 5632 18.9, 19.1.  32 x 32: 512^3 4.1, 4.7.
-// 128 x 128: 1536^2 x 4096 35.1, 37.)
+// 128 x 128: 1536^2 x 4096 35.1, 37.  30 other products, of the kernel each
+// chose: 0.71 to 1.50 of the estimate, median 1.01; profiles/tile_estimates.txt.)
 static double tile_us(int bm, int bn, long long tiles, long long ks, long long kbytes, long long es, int out_bytes, int cus) {
   const bool bytes = es == 1;
   double start, rate;  // us a round; KB of operands a us

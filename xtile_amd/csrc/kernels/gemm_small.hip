@@ -4,9 +4,13 @@
 // rows, 1024^3), whose M or N no 128-wide tile divides, or whose sizes or
 // alignment the DMA kernel of gemm.hip does not take at all.
 //
-// What bounds such a launch is how fast one CU gets its operands: ~55 bytes a
-// clock through the address unit, behind a latency of 1-2 us, against little
-// matrix work.  So the kernel keeps as many bytes in flight as LDS holds, and
+// What bounds such a launch is how fast one CU gets its operands, behind the
+// start and end of a launch, against little matrix work: beyond about 6 us the
+// time grows by 72 KB of operands a us and CU at 64 x 64 tiles of f16, by 36 at
+// 32 x 32 of i8, whose 32-byte rows of B make four requests of a line (1024^3:
+// 0.52 M requests to L2, matrix pipes busy 0.11 of its cycles;
+// 64 x 4096 x 4096 i8: 1.31 M requests, 0.80 of them B's, busy 0.04;
+// profiles/small_gemm_rates.txt, matmul_*_gemm_small.txt).  So the kernel keeps as many bytes in flight as LDS holds, and
 // nothing waits for anything else: the workgroup's four waves split K between
 // them (stage s of 64 K bytes belongs to wave s % 4), each wave fills its own
 // LDS ring, waits for its own loads and multiplies the whole BM x BN tile, so
