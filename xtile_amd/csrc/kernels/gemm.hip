@@ -523,17 +523,22 @@ static int cu_count() {
 // 128 x 128: 1536^2 x 4096 35.1, 37.  30 other products, of the kernel each
 // chose: 0.71 to 1.50 of the estimate, median 1.01; profiles/tile_estimates.txt.)
 static double tile_us(int bm, int bn, long long tiles, long long ks, long long kbytes, long long es, int out_bytes, int cus) {
+  const double n = double(tiles) * ks / cus;
+  // K split: start, end and the zero fill, a range's operands, the atomic sums;
+  // 660 products of 256 x 256 to 1024 x 2048 outputs, 2 to 16 ranges: 0.94 to 1.15
+  // of it (256 x 512 x 8192 in 16 ranges 15.1 us, 32 x 32 tiles 22.3)
+  if (ks > 1)
+    return 3.65 + std::ceil(n) * (bm + bn) * kbytes / ks / 1024 / 59 + 3.9 * ks * double(tiles) * bm * bn / (1 << 20);
   const bool bytes = es == 1;
   double start, rate;  // us a round; KB of operands a us
-  if (bm >= 128) start = bm == 256 ? 3 : 2.5, rate = ks > 1 || bm == 256 ? 50 : 62;
+  if (bm >= 128) start = bm == 256 ? 3 : 2.5, rate = bm == 256 ? 50 : 62;
   else if (bm == 64) start = 3.2, rate = bytes ? 60 : 70;
   else if (bn == 64) start = 2.1, rate = bytes ? 55 : 70;
   else start = 1.5, rate = bytes ? 36 : 50;  // a row of B is a quarter or half of a cache line
-  const double round = start + double(bm + bn) * kbytes / ks / 1024 / rate + double(bm) * bn * out_bytes / 1024 / 30;
-  const double n = double(tiles) * ks / cus;
+  const double round = start + double(bm + bn) * kbytes / 1024 / rate + double(bm) * bn * out_bytes / 1024 / 30;
   // 128 x 128 tiles run two to a CU, the others one
   const double rounds = bm >= 128 && bm + bn < 512 && n > 2 ? n : std::ceil(n);
-  return 1.8 + rounds * round + (ks > 1 ? 2.8 + 2.0 * ks : 0);  // the zero fill, the atomic sums
+  return 1.8 + rounds * round;
 }
 
 // Tiles of bm x bn over the plan's whole M x N region, columns along x, rows
