@@ -44,7 +44,8 @@ def run_gpu(module, host_buffers, dtypes, device, func=None, case: str = "", ker
     torch.cuda.synchronize()
     got = [to_host(t, d) for t, d in zip(dev, dtypes)]
     if kernels is not None:
-        assert kernels_of(module, dev, func) == kernels
+        ran = kernels_of(module, dev, func)
+        assert ran == kernels, ran
     return got
 
 

@@ -58,6 +58,10 @@ def _igemm(dt, bm, bn, part=0, split=False):
     return ["ig_zero_kernel"] * split + [f"conv_igemm_kernel<{_ELEM[dt]}, {bm}, {bn}, {rest}, {part}, 4>"]
 
 
+def _deep(dt, split=False):
+    return ["ig_zero_kernel"] * split + [f"conv_igemm_kernel<{_ELEM[dt]}, 64, 128, 32, 64, 128, 8, 0, 4>"]
+
+
 # (layer), the kernel of its own choice, the one with XTILE_AMD_CONV_IGEMM=1
 _LAYERS = [
     ((1, 1, 1, 512, 8, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "f16"),        # one pixel, one stage of 8 channels
@@ -90,6 +94,10 @@ _LAYERS = [
      _tiles("i8", 32, 64, 1), _igemm("i8", 128, 64, 1)),
     ((19, 112, 112, 20, 16, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),
      ["conv2d_small_kernel<2, 0, 0, 0>"], _igemm("i8", 256, 64, 1)),
+    ((2, 11, 11, 512, 512, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "f16"),    # 64 x 128 tiles, their K split
+     _deep("f16", split=True), None),
+    ((20, 17, 17, 256, 256, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),    # whole
+     _deep("i8"), None),
     ((2, 65, 65, 16, 128, 1, 1, (0, 0, 0, 0), (2, 2), (1, 1), "bf16"),
      _tiles("bf16", 32, 64), None),
     ((7, 24, 24, 16, 96, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),
@@ -105,17 +113,18 @@ _LAYERS = [
 ]
 
 
-@pytest.mark.parametrize("layer,kernels", [(x, own) for x, own, _ in _LAYERS] + [(x, forced) for x, _, forced in _LAYERS if forced])
-def test_conv_tiles(cuda, monkeypatch, layer, kernels):
+@pytest.mark.parametrize("layer,kernels,forced", [(x, own, False) for x, own, _ in _LAYERS] +
+                         [(x, igemm, True) for x, _, igemm in _LAYERS if igemm])
+def test_conv_tiles(cuda, monkeypatch, layer, kernels, forced):
     monkeypatch.setenv("XTILE_AMD_CONV_IMAGE", "0")
-    if "igemm" in kernels[-1]:
+    if forced:
         monkeypatch.setenv("XTILE_AMD_CONV_IGEMM", "1")
     _conv(cuda, *layer, kernels)
 
 
 @pytest.mark.parametrize(
     "n,h,cin,cout,k,pad,stride,dt,kernels",
-    [(20, 28, 128, 128, 3, 1, 1, "f16", _igemm("f16", 128, 64)),      # two stages a tap
+    [(20, 28, 128, 128, 3, 1, 1, "f16", _deep("f16")),                # two stages a tap
      (32, 28, 128, 128, 3, 1, 1, "f16", _igemm("f16", 128, 128)),
      (17, 37, 136, 96, 3, 1, 1, "bf16", _igemm("bf16", 128, 128)),    # channels past Cout, stages past a tap's channels
      (13, 47, 96, 64, 5, 2, 2, "f16", _igemm("f16", 256, 64, split=True)),  # pixels past the last tile
@@ -126,7 +135,7 @@ def test_conv_tiles(cuda, monkeypatch, layer, kernels):
      (32, 28, 132, 128, 3, 1, 1, "i8", _igemm("i8", 128, 128, 1))],   # of 4 channels
 )
 def test_conv_loader_waves(cuda, monkeypatch, n, h, cin, cout, k, pad, stride, dt, kernels):
-    """conv_igemm.hip's 128 x 128 and 128 x 64 tiles with loader waves, and the
-    split that one of the layers takes instead."""
+    """conv_igemm.hip's 128 x 128 and 128 x 64 tiles with loader waves, and the 64 x
+    128 tiles and the split that two of the layers take instead."""
     monkeypatch.setenv("XTILE_AMD_CONV_IGEMM", "1")
     _conv(cuda, n, h, h, cin, cout, k, k, (pad,) * 4, (stride, stride), (1, 1), dt, kernels)
