@@ -98,6 +98,10 @@ _LAYERS = [
      _deep("f16", split=True), None),
     ((20, 17, 17, 256, 256, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "i8"),    # whole
      _deep("i8"), None),
+    ((50, 40, 40, 96, 64, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "bf16"),    # bands of four rows, half the filter's bytes
+     ["conv2d_band_kernel<2, 6, 1>"], None),
+    ((53, 21, 21, 64, 128, 3, 3, (1, 1, 1, 1), (1, 1), (1, 1), "f16"),    # of two rows, a tenth of them
+     _igemm("f16", 128, 128), None),
     ((2, 65, 65, 16, 128, 1, 1, (0, 0, 0, 0), (2, 2), (1, 1), "bf16"),
      _tiles("bf16", 32, 64), None),
     ((7, 24, 24, 16, 96, 1, 1, (0, 0, 0, 0), (1, 1), (1, 1), "i8"),

@@ -787,7 +787,8 @@ int ilog2(unsigned v) {
 // every Block uses one filter.  Returns false (nothing launched) when
 // it does not apply; `e` carries a launch error otherwise.
 // `thin`: also bands that the filter leaves LDS for at most half the rows of an
-// even split, of less than half the filter's bytes.
+// even split, of less than half the filter's bytes (a quarter for several rows at
+// stride 1, which share their halo).
 bool try_band(const xt::Plan& p, void* const* bufs, hipStream_t s, int max_lds, int cus, bool thin, hipError_t& e) {
   const xt::ConvPlan& c = p.conv;
   if (c.cb.axis < 0 || c.ch.axis < 0 || c.cw.axis < 0 || c.cb.axis == c.ch.axis || c.cb.axis == c.cw.axis ||
@@ -851,7 +852,7 @@ bool try_band(const xt::Plan& p, void* const* bufs, hipStream_t s, int max_lds, 
       break;
     }
   }
-  if (R < 1 || (!thin && R * 2 <= even && filt_bytes > 2 * hrows_max * rpitch)) return false;
+  if (R < 1 || (!thin && R * 2 <= even && filt_bytes > (R == 1 || c.stride_h > 1 ? 2 : 4) * hrows_max * rpitch)) return false;
   // the kernel divides pixel indices below 2^16 by multiply-high reciprocals
   if (hrows_max * ipr >= 65536 || R * c.out_W >= 65536 || rf_w >= 65536 || c.out_W >= 65536) return false;
   if (R * c.out_W * c.CO * 4 >= (1LL << 31)) return false;
@@ -992,7 +993,12 @@ hipError_t launch_conv2d(const xt::Plan& p, void* const* bufs, hipStream_t s, st
   // the filter's, come behind the implicit GEMM, which takes nearly every plan
   // that bands do (32 x 28^2 x 128 -> 128 i8, a 147 KB filter, bands of one row
   // for four: 16.2 us against 10.2; 64 x 112^2 x 32 -> 128 / 2 f16, a 73 KB
-  // filter, bands of four rows and 81 KB for fourteen: 37.4 against 42.5).
+  // filter, bands of four rows and 81 KB for fourteen: 37.4 against 42.5).  Of
+  // several rows at stride 1 only where the filter is most of the load by far: two of 13 KB
+  // beside 144 KB, 53 x 21^2 x 64 -> 128 f16, 14.7 against 10.1; but four of 51 KB
+  // beside 108, 50 x 40^2 x 96 -> 64 bf16, 15.5 against 23.8, and of 46 KB at stride
+  // 2, 64 x 43^2 x 96 -> 64 f16, 16.1 against 12.6 (of 61 such layers drawn 8 were
+  // slower behind the implicit GEMM at a factor of two throughout, 1 is now).
   if (try_band(p, bufs, s, max_lds, cus, false, e)) return e;
   // filters beyond the band kernel's LDS: each image resident in LDS when
   // its channels fit there, else the implicit GEMM with DMA operands
