@@ -63,6 +63,20 @@ def test_row_softmax(cuda, rows, cols, trow, off):
     np.testing.assert_allclose(got, closed_form.softmax_rows(x), rtol=1e-5, atol=1.2e-38)
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("rows,cols,trow,groups", [(512, 1025, 1, "2, 256"), (513, 1025, 1, "5, 64"), (514, 1536, 2, "6, 64"),
+                                                  (520, 1790, 4, "7, 64"), (516, 2047, 3, "8, 64"), (512, 2047, 4, "2, 256"),
+                                                  (513, 1024, 1, "4, 64"), (5, 1024, 1, "4, 64")])
+def test_few_long_rows(cuda, rows, cols, trow, groups, off):
+    """Up to 512 rows of 1025 to 2048 floats take the workgroup, more a wave."""
+    rng = np.random.default_rng(rows + cols)
+    x = rng.normal(0, 2, (rows, cols)).astype(np.float32)
+    m = K.softmax(rows, cols, trow)
+    got = _run(cuda, m, off, f"softmax {rows}x{cols}/{trow}", x, np.zeros_like(x))
+    np.testing.assert_allclose(got, closed_form.softmax_rows(x), rtol=1e-5, atol=1.2e-38)
+    assert kernels_of(m, _views(cuda, off, x, np.zeros_like(x))[1]) == [f"row_softmax_kernel<{groups}, 0>"]
+
+
 @pytest.mark.parametrize("rows,cols,trow,kernel", [((1 << 32) + 4096, 2, 4096, "row_softmax_kernel<1, 1, 1>"),
                                                   (8388611, 2048, 7, "row_softmax_wide_kernel<512, 1, 1>")])
 def test_row_softmax_of_more_rows_than_a_launch_takes(cuda, rows, cols, trow, kernel):

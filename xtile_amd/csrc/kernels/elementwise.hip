@@ -466,12 +466,14 @@ hipError_t launch_row_softmax(const xt::Plan& p, void* const* bufs, hipStream_t 
   const bool vec = aligned4(p.a, a.x) && aligned4(p.c, a.y);
   const long long blocks = grid_blocks(p), total = blocks * a.rows;
   const bool wide = vec && a.cols % 2048 == 0 && a.cols <= 8 * 2048;
-  // threads a row: a power of two up to a wave for rows up to 2048 floats, else
-  // the workgroup; two float4 a thread where that makes it less than a wave and
+  // threads a row: a power of two up to a wave for rows up to 2048 floats, else,
+  // and where there are so few that a wave's eight float4 are latency (64 x 2000
+  // 4.0 us a wave each, 3.7 a workgroup; 1024 x 2000 5.0 either way; to 1024
+  // floats no different), the workgroup; two float4 a thread where that makes it less than a wave and
   // there are rows to fill the chip all the same (100000 x 100: 43.7 -> 17.0 us;
   // 64 x 256 2.5 with two, 2.3 with one)
   int tpr = 256;
-  if (a.cols <= 2048)
+  if (a.cols <= 1024 || (a.cols <= 2048 && total > 512))
     for (tpr = 1; tpr < 64 && tpr * (total > 4096 ? 8 : 4) < a.cols; tpr *= 2) {
     }
   const int threads = wide ? 512 : 256;
