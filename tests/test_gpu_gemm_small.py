@@ -76,7 +76,7 @@ _SPLIT = ["gemm_zero_kernel", "gemm_dma_kernel<0, 4, 0, 0, 4, 1, 128, 128, 0>"]
      ("bf16", 2112, 4160, 320, 64, 64, "gemm", _edge("bf16", 128)),             # M and N edges
      ("f16", 256, 512, 8192, 128, 64, "gemm", _SPLIT),                          # 8 tiles in 16 K ranges
      ("f16", 256, 256, 5376, 64, 64, "gemm", _SPLIT),
-     ("f16", 256, 256, 2048, 64, 64, "gemm", _small("f16", 32, 32, _DMA)),
+     ("f16", 256, 256, 2560, 64, 64, "gemm", _small("f16", 32, 32, _DMA)),
      ("f16", 1600, 6656, 512, 64, 128, "gemm", _edge("f16", 256)),              # M edge
      ("bf16", 4864, 2112, 256, 128, 64, "gemm", _edge("bf16", 256))],           # N edge
 )
