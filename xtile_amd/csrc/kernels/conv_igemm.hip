@@ -557,14 +557,15 @@ bool conv_blocks_cover_output(const xt::Plan& p, long long es) {
 // to 124509 x 16.  Here a stage took 0.44 us whatever the tile while a CU has one
 // workgroup, and a launch 5.2, a K split 2.5 for the zero fill and 2 a million
 // atomic sums; the 64 x 128 tiles (deep) 4.4 and 0.32, split 4.6, 0.39 and 2.75 a
-// million (2864 layers, 0.88 to 1.08 of it for nine of ten; at the others' figures
-// they stood 15% too high, and 493 of 4052 such layers went to tiles that took up
-// to 23% longer, 2 x 11^2 x 512 -> 512 3 x 3 f16 12.5 -> 15.1); there a round of tiles costs its start
+// million (1759 layers, 0.93 to 1.15 of it for nine of ten; at the others' figures
+// they stood 15% too high, and 227 of those layers went to tiles that took 5 to
+// 23% longer, 2 x 11^2 x 512 -> 512 3 x 3 f16 12.5 -> 15.1;
+// profiles/dispatch_rules.txt); there a round of tiles costs its start
 // and end and its operands at ~70 KB a us.  (Measured / estimated: 5 x 18^2 x 512
 // -> 32 3 x 3 / 2 i8 36.6 / 36.9 here, 7.1 / 7.7 in 32 x 32 tiles; 53 x 47^2 x 40
 // -> 64 5 x 5 / 2 30.6 / 26.5, 15.3 / 14.9 in 64 x 64; 32 x 28^2 x 128 -> 128 20.1
 // / 21.0, 30.8 / 26.9.  40 other layers, of the kernel each chose, loader-wave
-// tiles among them: 0.86 to 1.34, median 0.98; profiles/tile_estimates.txt.)
+// tiles among them: 0.86 to 1.37, median 0.99; profiles/tile_estimates.txt.)
 static double igemm_us(bool deep, int stages, long long nwg, long long ksplit, long long outputs, int cus) {
   const double load = std::max(1.0, 0.85 * double(nwg) / cus), sums = 1e-6 * outputs * ksplit;
   if (deep) return ksplit > 1 ? 4.6 + 0.39 * stages / ksplit * load + 2.75 * sums : 4.4 + 0.32 * stages * load;

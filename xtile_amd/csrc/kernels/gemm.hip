@@ -521,12 +521,13 @@ static int cu_count() {
 // (64 x 64: 1024^3 f16 9.5 us measured, 9.2 estimated; 1024 x 1024 x 4096 21.0,
 // 20.1.  32 x 64: 256 x 2048 x 5632 18.9, 19.1.  32 x 32: 512^3 4.1, 4.7.
 // 128 x 128: 1536^2 x 4096 35.1, 37.  30 other products, of the kernel each
-// chose: 0.71 to 1.50 of the estimate, median 1.01; profiles/tile_estimates.txt.)
+// chose: 0.71 to 1.53 of the estimate, median 1.01; profiles/tile_estimates.txt.)
 static double tile_us(int bm, int bn, long long tiles, long long ks, long long kbytes, long long es, int out_bytes, int cus) {
   const double n = double(tiles) * ks / cus;
   // K split: start, end and the zero fill, a range's operands, the atomic sums;
-  // 660 products of 256 x 256 to 1024 x 2048 outputs, 2 to 16 ranges: 0.94 to 1.15
-  // of it (256 x 512 x 8192 in 16 ranges 15.1 us, 32 x 32 tiles 22.3)
+  // 1075 products of 256 x 256 to 1536 x 1280 outputs, 2 to 16 ranges: 0.90 to 1.18
+  // of it (256 x 512 x 8192 in 16 ranges 15.1 us, 32 x 32 tiles 22.3;
+  // profiles/dispatch_rules.txt)
   if (ks > 1)
     return 3.65 + std::ceil(n) * (bm + bn) * kbytes / ks / 1024 / 59 + 3.9 * ks * double(tiles) * bm * bn / (1 << 20);
   const bool bytes = es == 1;
